@@ -51,6 +51,9 @@ struct GemmParams {
     // tile order: bands of group_m tile rows, each band walked column by column (1: row
     // major); each XCD then takes a contiguous run of that order (tile_coords)
     int group_m;
+    // 1: [rows] x [out][in]^T products with MFMA chains of at most 64 k where gemm_bl_kernel
+    // takes them (64x64 tiles only); see there
+    int short_chains;
 };
 
 // The first kSplitCounterBytes of a split-K workspace hold the per-tile arrival counters of

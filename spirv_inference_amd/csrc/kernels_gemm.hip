@@ -635,7 +635,11 @@ __device__ __host__ inline int64_t bl_b_extent(const GemmParams& p, int bmode) {
     return (int64_t)(p.K - 1) * p.sbk + p.N;
 }
 
-template <int BM, int BN, int BK, int AM, int BMD>
+//
+// FL cuts the MFMA chains every 64 k (32 with the 16-deep tile) and adds them to a second
+// accumulator set, for callers whose sums must not lose to a vector-unit reduction (the decoder's
+// prompt pass against its token steps): 3 % more issue slots.
+template <int BM, int BN, int BK, int AM, int BMD, bool FL = false>
 __global__ __launch_bounds__(256) void gemm_bl_kernel(GemmParams p) {
     static_assert(AM == shp::A_KVEC || AM == shp::A_CONV_NHWC4, "row-contiguous A");
     static_assert(BMD == shp::B_NVEC || BMD == shp::B_KVEC, "row-contiguous B");
@@ -749,13 +753,29 @@ __global__ __launch_bounds__(256) void gemm_bl_kernel(GemmParams p) {
         }
     };
 
-    floatx16 acc[FM][FN];
+    floatx16 acc[FM][FN], sum[FL ? FM : 1][FL ? FN : 1];
 #pragma unroll
     for (int i = 0; i < FM; ++i)
 #pragma unroll
         for (int j = 0; j < FN; ++j)
 #pragma unroll
-            for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.0f;
+            for (int r = 0; r < 16; ++r) {
+                acc[i][j][r] = 0.0f;
+                if constexpr (FL) sum[i][j][r] = 0.0f;
+            }
+    auto flush = [&]() __attribute__((always_inline)) {
+        if constexpr (FL) {
+#pragma unroll
+            for (int i = 0; i < FM; ++i)
+#pragma unroll
+                for (int j = 0; j < FN; ++j)
+#pragma unroll
+                    for (int r = 0; r < 16; ++r) {
+                        sum[i][j][r] += acc[i][j][r];
+                        acc[i][j][r] = 0.0f;
+                    }
+        }
+    };
 
     // Fragments of one step: lanes 0-31 feed k = s of the tile, lanes 32-63 k = BK/2 + s (A and
     // B agree, so any assignment of the tile's k to MFMA k-pairs works), so each lane reads four
@@ -828,15 +848,23 @@ __global__ __launch_bounds__(256) void gemm_bl_kernel(GemmParams p) {
         int kt = 0;
         for (; kt + 1 < ntk; kt += 2) {
             tile(0, s1, true, s0, min(kt + 2, ntk - 1));
+            if constexpr (BK == 64) flush();
             __syncthreads();
             tile(1, s0, kt + 2 < ntk, s1, min(kt + 3, ntk - 1));
+            flush();
             __syncthreads();
         }
         if (kt < ntk) {
             tile(0, s1, false, s0, kt);
+            flush();
             __syncthreads();
         }
     }
+    if constexpr (FL)
+#pragma unroll
+        for (int i = 0; i < FM; ++i)
+#pragma unroll
+            for (int j = 0; j < FN; ++j) acc[i][j] = sum[i][j];
 
     gemm_epilogue<BM, BN, 2, 2, RC, CS, shp::C_STRIDED>(p, acc, smem, m0, n0, split, p.splits, bz,
                                                         bo, bi, gridDim.z,
@@ -1988,6 +2016,17 @@ int bl_mask(const GemmParams& p, int am, int bm, int cm) {
 
 template <int AM, int BMD>
 void launch_bl_combo(hipStream_t s, const GemmParams& p, TileCfg t, dim3 grid) {
+    if constexpr (AM == shp::A_KVEC && BMD == shp::B_KVEC) {
+        if (p.short_chains && t.bm == 64) {
+            if (t.bk == 64)
+                hipLaunchKernelGGL((gemm_bl_kernel<64, 64, 64, AM, BMD, true>), grid, dim3(256), 0, s, p);
+            else if (t.bk == 16)
+                hipLaunchKernelGGL((gemm_bl_kernel<64, 64, 16, AM, BMD, true>), grid, dim3(256), 0, s, p);
+            else
+                hipLaunchKernelGGL((gemm_bl_kernel<64, 64, 32, AM, BMD, true>), grid, dim3(256), 0, s, p);
+            return;
+        }
+    }
     if (t.bm == 128 && t.bn == 128)
         hipLaunchKernelGGL((gemm_bl_kernel<128, 128, 32, AM, BMD>), grid, dim3(256), 0, s, p);
     else if (t.bm == 128)
@@ -2237,6 +2276,7 @@ bool plan_bl(const GemmParams& p, int nbatch, int blm, const shp::GemmTune& tn, 
         const int ti = t.bm == 128 ? (t.bn == 128 ? 1 : 2) : 3;
         if (tn.tile && tn.tile != ti) continue;
         if (tn.bk && tn.bk != t.bk) continue;
+        if (p.short_chains && t.bm == 128) continue;
         const int kq = t.bk == 64 ? 64 : 32;
         for (int s : kSplits) {
             if (tn.splits && tn.splits != s) continue;

@@ -11,9 +11,13 @@
 // decode call as one cooperative launch (kernels_decode_persist.hip).  Nothing returns to
 // the host between tokens in either form.
 #include <cmath>
+#include <cstring>
 #include <vector>
 
+#include "attention.h"
 #include "decode.h"
+#include "gemm.h"
+#include "prefill.h"
 #include "runtime.h"
 
 namespace shp {
@@ -249,6 +253,146 @@ struct Llama {
         return SHP_OK;
     }
 
+    // ---- prompt pass: positions in chunks of up to pf_rows -----------------------------------
+    int pf_rows = 0;         // 0: the shape is outside the prompt kernels' limits
+    int pf_logit_rows = 0;   // rows of logits computed at once
+    float *pf_x = nullptr, *pf_h = nullptr, *pf_q = nullptr, *pf_att = nullptr;
+    float *pf_sum = nullptr;     // product results or K-split partials
+    float *pf_act = nullptr, *pf_logits = nullptr;
+
+    GemmParams product(int rows, const float* a, const float* w, int N, int K, float* c,
+                       const float* residual) const {
+        GemmParams p;
+        std::memset(&p, 0, sizeof p);
+        p.batch_outer = p.batch_inner = 1;
+        p.coh = p.cow = p.splits = 1;
+        p.M = rows; p.N = N; p.K = K;
+        p.a = a; p.sam = K; p.sak = 1;
+        p.b = w; p.sbk = 1; p.sbn = K;
+        p.c = c; p.scm = N; p.scn = 1;
+        p.residual = residual;
+        p.short_chains = 1;
+        return p;
+    }
+    int tiled(int rows, const float* a, const float* w, int N, int K, float* c,
+              const float* residual = nullptr) {
+        const GemmParams p = product(rows, a, w, N, K, c, residual);
+        int rc = ctx->ensure_workspace(gemm_workspace_bytes(p, A_KVEC, B_KVEC, C_STRIDED, &ctx->tune));
+        if (rc) return rc;
+        return gemm_launch(ctx->stream, p, A_KVEC, B_KVEC, C_STRIDED, ctx->workspace,
+                           ctx->workspace_bytes, &ctx->tune);
+    }
+
+    // Buffers of the prompt pass, kept with the decoder: 0.12 MB per position at TinyLlama's
+    // shape, at most 512 positions.
+    int setup_prefill() {
+        const uint64_t H = cfg.hidden, F = cfg.ffn, qd = (uint64_t)cfg.n_heads * 64;
+        const uint64_t widest = std::max<uint64_t>(2 * F, std::max<uint64_t>(cfg.vocab, qkv_rows()));
+        const uint64_t deepest = std::max(std::max(H, F), qd);
+        if (cfg.max_seq < 2 || H % 8 || cfg.vocab % 8 || F % 4 ||
+            widest * deepest * 4 >= (1ull << 31))
+            return SHP_OK;
+        const int rows = std::min(cfg.max_seq, kPrefillRows);
+        const uint64_t R = rows, skinny = std::min(rows, kSkinnyRows);
+        int rc = alloc(&pf_x, R * H);
+        if (!rc) rc = alloc(&pf_h, R * H);
+        if (!rc) rc = alloc(&pf_q, R * qd);
+        if (!rc) rc = alloc(&pf_att, R * qd);
+        if (!rc) rc = alloc(&pf_act, R * F);
+        if (!rc)
+            rc = alloc(&pf_sum, std::max(R * std::max<uint64_t>(2 * F, qkv_rows()),
+                                         skinny * kSkinnySplits * std::max<uint64_t>(H, qkv_rows())));
+        pf_logit_rows = std::min(rows, 128);
+        if (!rc) rc = alloc(&pf_logits, (uint64_t)pf_logit_rows * cfg.vocab);
+        if (!rc) pf_rows = rows;
+        return rc;
+    }
+
+    // Positions host_pos .. host_pos + n - 1 of a prompt (n <= pf_rows): appends their keys and
+    // values, logs every position's argmax and leaves the last one's logits and token as a step
+    // at that position would.
+    int prefill_chunk(const int32_t* prompt, int n) {
+        const int H = cfg.hidden, F = cfg.ffn, qd = cfg.n_heads * 64, QR = qkv_rows();
+        const uint64_t cache_layer = (uint64_t)cfg.n_kv_heads * cfg.max_seq * cfg.head_dim;
+        const bool skinny = n <= kSkinnyRows;
+        hipStream_t s = ctx->stream;
+        PrefillIds ids;
+        std::memcpy(ids.id, prompt, (size_t)n * sizeof(int32_t));
+        const int sp_qkv = skinny ? skinny_splits(QR, H) : 1;
+        const int sp_wo = skinny ? skinny_splits(H, qd) : 0;
+        const int sp_down = skinny ? skinny_splits(H, F) : 0;
+        int rc = prefill_embed_launch(s, embed, H, ids, n, pf_x);
+        for (int l = 0; l < cfg.n_layers && !rc; ++l) {
+            const Layer& L = layers[l];
+            float* kc = k_cache + l * cache_layer;
+            float* vc = v_cache + l * cache_layer;
+            // the partials of the layer before's down product are added where its sum is read
+            rc = prefill_norm_launch(s, pf_x, pf_sum, l ? sp_down : 0, pf_x, L.attn_norm,
+                                     cfg.rms_eps, pf_h, n, H);
+            if (!rc)
+                rc = skinny ? skinny_launch(s, pf_h, n, L.wqkv, QR, H, SK_PARTIAL, sp_qkv, pf_sum)
+                            : tiled(n, pf_h, L.wqkv, QR, H, pf_sum);
+            if (!rc)
+                rc = prefill_rope_launch(s, pf_sum, sp_qkv, pf_q, kc, vc, n, cfg.n_heads,
+                                         cfg.n_kv_heads, cfg.max_seq, host_pos, cfg.rope_theta);
+            if (!rc) {
+                AttnArgs a{};
+                a.q = pf_q; a.k = kc; a.v = vc; a.out = pf_att;
+                a.q_h = 64; a.q_r = qd; a.o_h = 64; a.o_r = qd;
+                a.k_h = a.v_h = (int64_t)cfg.max_seq * 64;
+                a.k_r = a.v_r = 64;
+                a.batch = 1;
+                a.kv_heads = cfg.n_kv_heads;
+                a.group = cfg.n_heads / cfg.n_kv_heads;
+                a.n_queries = n;
+                a.n_keys = host_pos + n;
+                a.causal = 1;
+                a.pos0 = host_pos;
+                a.scale = 0.125f;
+                rc = attention_launch(s, a);
+            }
+            if (!rc)
+                rc = skinny ? skinny_launch(s, pf_att, n, L.wo, H, qd, SK_PARTIAL, sp_wo, pf_sum)
+                            : tiled(n, pf_att, L.wo, H, qd, pf_x, pf_x);
+            if (!rc)
+                rc = prefill_norm_launch(s, pf_x, pf_sum, sp_wo, pf_x, L.ffn_norm, cfg.rms_eps,
+                                         pf_h, n, H);
+            if (skinny) {
+                if (!rc) rc = skinny_launch(s, pf_h, n, L.w_gu, 2 * F, H, SK_SWIGLU, 1, pf_act);
+                if (!rc)
+                    rc = skinny_launch(s, pf_act, n, L.w_down, H, F, SK_PARTIAL, sp_down, pf_sum);
+            } else {
+                if (!rc) rc = tiled(n, pf_h, L.w_gu, 2 * F, H, pf_sum);
+                if (!rc) rc = prefill_swiglu_launch(s, pf_sum, pf_act, n, F);
+                if (!rc) rc = tiled(n, pf_act, L.w_down, H, F, pf_x, pf_x);
+            }
+        }
+        if (!rc)
+            rc = prefill_norm_launch(s, pf_x, pf_sum, sp_down, pf_x, final_norm, cfg.rms_eps, pf_h,
+                                     n, H);
+        for (int r = 0; r < n && !rc; r += pf_logit_rows) {
+            const int m = std::min(pf_logit_rows, n - r);
+            const float* h = pf_h + (uint64_t)r * H;
+            rc = m <= kSkinnyRows
+                     ? skinny_launch(s, h, m, lm_head, cfg.vocab, H, SK_PARTIAL, 1, pf_logits)
+                     : tiled(m, h, lm_head, cfg.vocab, H, pf_logits);
+            if (!rc)
+                rc = prefill_argmax_launch(s, pf_logits, m, cfg.vocab, st->out_tokens + host_pos + r,
+                                           r + m == n ? logits : nullptr, &st->token, &st->pos,
+                                           &st->step, host_pos + n);
+        }
+        if (!rc) host_pos += n;
+        return rc;
+    }
+
+    // A whole prompt from position 0 (after reset()).
+    int prefill(const int32_t* prompt, int n) {
+        int rc = check_room(n);
+        for (int i = 0; i < n && !rc; i += pf_rows)
+            rc = prefill_chunk(prompt + i, std::min(pf_rows, n - i));
+        return rc;
+    }
+
     int reset() {
         SHP_HIP_CHECK(hipMemsetAsync(st, 0, sizeof(DecodeState), ctx->stream));
         host_pos = 0;
@@ -316,6 +460,7 @@ int shp_llama_create(shp_ctx* ctx, const shp_llama_config* cfg, uint64_t seed, s
     }
     if (!rc) rc = lm->reset();
     if (!rc) rc = lm->setup_persistent();
+    if (!rc) rc = lm->setup_prefill();
     if (!rc && lm->p_grid > 0) lm->engine = SHP_LLAMA_PERSISTENT;
     if (!rc) {
         hipError_t e = hipStreamSynchronize(lm->ctx->stream);
@@ -404,7 +549,14 @@ int shp_llama_generate(shp_llama* p, const int32_t* prompt, int32_t n_prompt, in
     if (n_prompt + n_new - 1 > lm->cfg.max_seq)
         return fail(SHP_ERR_SHAPE, "shp_llama_generate: prompt + new tokens exceed max_seq");
     int rc = lm->reset();
-    for (int i = 0; i < n_prompt && !rc; ++i) rc = shp_llama_step(p, prompt[i]);
+    if (n_prompt > 1 && lm->pf_rows) {
+        for (int i = 0; i < n_prompt && !rc; ++i)
+            if (prompt[i] < 0 || prompt[i] >= lm->cfg.vocab)
+                rc = fail(SHP_ERR_SHAPE, "shp_llama_step: token id");
+        if (!rc) rc = lm->prefill(prompt, n_prompt);
+    } else {
+        for (int i = 0; i < n_prompt && !rc; ++i) rc = shp_llama_step(p, prompt[i]);
+    }
     if (!rc && n_new > 1) rc = shp_llama_decode(p, n_new - 1);
     if (rc) return rc;
     std::vector<int32_t> all(4096);

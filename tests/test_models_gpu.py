@@ -298,6 +298,48 @@ def test_llama_small_tokens_and_logits(ctx, orc, engine):
         assert lm.generate(prompt, 8) == (want[:stop[0]] if stop else want)
 
 
+@pytest.mark.parametrize("n", [2, 15, 16, 17, 33, 64, 65, 130, 512, 513, 600])
+def test_llama_prompt_pass_equals_token_steps(ctx, n):
+    """generate() takes the whole prompt in one pass (up to 64 rows per product on the
+    weight-streaming kernel, above on the tiled ones, 512 positions per chunk); the argmax of every
+    position, the KV cache and the last logits equal those of the prompt fed one step per id."""
+    from spirv_inference_amd.models import Llama
+    cfg = dict(SMALL, max_seq=640, ffn=520, vocab=1016)
+    rng = np.random.default_rng(n)
+    prompt = [int(t) for t in rng.integers(3, cfg["vocab"], n)]
+    with Llama(ctx, seed=9, **cfg) as lm:
+        lm.reset()
+        for t in prompt:
+            lm.step(t)
+        lm.decode(2)
+        ctx.sync()
+        rows = (n + 2) * 64
+
+        def state():
+            out = {"logits": lm.logits()}
+            for layer in range(cfg["n_layers"]):
+                for which in ("k_cache", "v_cache"):
+                    c = lm.weight(layer, which).reshape(cfg["n_kv_heads"], -1)
+                    out[f"{which}{layer}"] = c[:, :rows]
+            return out
+
+        tokens, want = lm.tokens(), state()
+        lm.generate(prompt, 3)
+        assert lm.tokens() == tokens
+        got = state()
+        for k, w in want.items():
+            assert_close(got[k].ravel(), w.ravel(), 1e-4, 1e-4, f"prompt of {n}: {k}")
+
+
+def test_llama_generate_refuses_bad_prompts(ctx):
+    from spirv_inference_amd import ShpError
+    from spirv_inference_amd.models import Llama
+    with Llama(ctx, seed=5, **SMALL) as lm:
+        for prompt, new in (([1, 1000], 2), ([-1, 5], 2), ([5] * 60, 6)):
+            with pytest.raises(ShpError, match="SHAPE"):
+                lm.generate(prompt, new)
+        assert len(lm.generate([5] * 60, 5)) <= 5
+
 def test_llama_kv_cache_matches_full_recompute(ctx, orc):
     """The oracle's KV-cache step equals the reference's algorithm (full causal recompute of
     every position, run_llama_spirv.py:198-206) on the same weights."""
