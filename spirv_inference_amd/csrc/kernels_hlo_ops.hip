@@ -18,6 +18,7 @@
 // element, consecutive threads on consecutive outputs.
 #include <cstring>
 
+#include "coherent.h"
 #include "common.h"
 
 namespace {
@@ -372,25 +373,41 @@ struct Red {
     int64_t rcount;
 };
 
+// Any reduced axes (after merging): one thread per output, the last reduced axis in batches of 16
+// loads that are all issued before the first of them is folded.
 __global__ __launch_bounds__(kBlock) void reduce_nd_kernel(const float* __restrict__ x,
                                                            float* __restrict__ y, Red p,
                                                            uint64_t total) {
+    constexpr int U = 16;
     const uint64_t stride = (uint64_t)gridDim.x * kBlock;
+    const int inner = p.rr ? p.rdims[p.rr - 1] : 1;
+    const int64_t step = p.rr ? p.rstride[p.rr - 1] : 0;
+    const int64_t outer = p.rcount / inner;
     for (uint64_t o = (uint64_t)blockIdx.x * kBlock + threadIdx.x; o < total; o += stride) {
         uint64_t rem = o;
-        int64_t base = 0;
+        int64_t off = 0;
         for (int k = p.rk - 1; k >= 0; --k) {
-            base += (int64_t)(rem % (uint64_t)p.kdims[k]) * p.kstride[k];
+            off += (int64_t)(rem % (uint64_t)p.kdims[k]) * p.kstride[k];
             rem /= (uint64_t)p.kdims[k];
         }
         float acc = p.init;
         int c[kMaxRank] = {0, 0, 0, 0, 0, 0, 0, 0};
-        int64_t off = base;
-        for (int64_t j = 0; j < p.rcount; ++j) {
-            const float v = x[off];
-            acc = p.kind ? fmaxf(acc, v) : acc + v;
+        for (int64_t j = 0; j < outer; ++j) {
+            const float* xp = x + off;
+            int i = 0;
+            for (; i + U <= inner; i += U) {
+                float v[U];
+#pragma unroll
+                for (int u = 0; u < U; ++u) v[u] = xp[(i + u) * step];
+#pragma unroll
+                for (int u = 0; u < U; ++u) acc = p.kind ? fmaxf(acc, v[u]) : acc + v[u];
+            }
+            for (; i < inner; ++i) {
+                const float v = xp[i * step];
+                acc = p.kind ? fmaxf(acc, v) : acc + v;
+            }
             // next reduced coordinate in row-major order (last reduced axis fastest)
-            for (int k = p.rr - 1; k >= 0; --k) {
+            for (int k = p.rr - 2; k >= 0; --k) {
                 off += p.rstride[k];
                 if (++c[k] < p.rdims[k]) break;
                 off -= (int64_t)p.rdims[k] * p.rstride[k];
@@ -399,6 +416,149 @@ __global__ __launch_bounds__(kBlock) void reduce_nd_kernel(const float* __restri
         }
         y[o] = acc;
     }
+}
+
+// Contiguous rows of n elements, one output per row.  The order of a sum is fixed (increasing
+// index), so an output's adds are one chain in one lane; what can be parallel is the memory.
+// 256 threads stage a tile of 8,192 floats, `rows` rows of 8192 / rows columns, with coalesced
+// loads into registers and then LDS (rows padded by 4 floats, so 16-byte reads down a column of
+// rows are free of bank conflicts), while the tile before it is folded by the first `rows`
+// threads.  Few rows per workgroup when there are few rows at all: 1,024 rows of 768 take four
+// each, one per CU, 114 us with a thread walking each row and 7.1 us so (10.5 before the LDS reads
+// were kept a batch ahead of the adds).
+constexpr int kRedTile = 8192;
+
+template <bool VEC, bool MAX>
+__global__ __launch_bounds__(256) void reduce_rows_kernel(const float* __restrict__ x,
+                                                          float* __restrict__ y,
+                                                          float init, int64_t nrows, int n,
+                                                          int rows) {
+    __shared__ __attribute__((aligned(16))) float tile[kRedTile + 256 * 4];
+    constexpr int W = VEC ? 4 : 1, NL = kRedTile / 256 / W;  // loads per thread and tile
+    const int tid = threadIdx.x;
+    const int cols = kRedTile / rows, ls = cols + 4;
+    const int64_t r0 = (int64_t)blockIdx.x * rows;
+    // Load i of a thread is a fixed distance from its load 0: a tile row is cols / W loads, a
+    // power of two, so 256 threads cover whole rows or a part of one.  No bounds checks: rows past
+    // the end are outside the buffer range, columns past n are never folded.
+    const int cw = cols / W, sh = 31 - __clz(cw);
+    const __amdgpu_buffer_rsrc_t xr = buffer_rsrc(x + r0 * n, min((int64_t)rows, nrows - r0) * n);
+    const int row = cw < 256 ? tid >> sh : 0, col = (cw < 256 ? tid & (cw - 1) : tid) * W;
+    const unsigned voff = (unsigned)(row * n + col) * 4u;
+    float* const lp = tile + row * ls + col;
+    float st[NL][W];
+    auto load = [&](int c0) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < NL; ++i) {
+            const int di = cw < 256 ? i * (256 >> sh) : (i * 256) >> sh;  // rows from load 0
+            const int dc = cw < 256 ? 0 : ((i * 256) & (cw - 1)) * W;
+            const unsigned so = (unsigned)(di * n + dc + c0) * 4u;
+            if constexpr (VEC) {
+                const f4v v = __builtin_bit_cast(f4v, __builtin_amdgcn_raw_buffer_load_b128(xr, voff, so, 0));
+                st[i][0] = v.x; st[i][1] = v.y; st[i][2] = v.z; st[i][3] = v.w;
+            } else {
+                st[i][0] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(xr, voff, so, 0));
+            }
+        }
+    };
+    load(0);
+    float acc = init;
+    for (int c0 = 0; c0 < n; c0 += cols) {
+        __syncthreads();  // the previous tile has been folded
+#pragma unroll
+        for (int i = 0; i < NL; ++i) {
+            const int di = cw < 256 ? i * (256 >> sh) : (i * 256) >> sh;
+            const int dc = cw < 256 ? 0 : ((i * 256) & (cw - 1)) * W;
+            float* d = lp + di * ls + dc;
+            if constexpr (VEC)
+                *reinterpret_cast<float4*>(d) = make_float4(st[i][0], st[i][1], st[i][2], st[i][3]);
+            else
+                *d = st[i][0];
+        }
+        __syncthreads();
+        if (c0 + cols < n) load(c0 + cols);
+        if (tid < rows) {
+            const float* t = tile + tid * ls;
+            const int m = min(cols, n - c0);
+            auto fold = [&](float4 v) __attribute__((always_inline)) {
+                if constexpr (MAX) {
+                    acc = fmaxf(fmaxf(fmaxf(fmaxf(acc, v.x), v.y), v.z), v.w);
+                } else {
+                    acc += v.x; acc += v.y; acc += v.z; acc += v.w;
+                }
+            };
+            // 32 elements at a time, the next 32 read while these are folded
+            int c = 0;
+            if (m >= 32) {
+                float4 a[8], b[8];
+                auto read = [&](float4 (&d)[8], int at) __attribute__((always_inline)) {
+                    const float* q = t + (at + 32 <= m ? at : 0);
+#pragma unroll
+                    for (int u = 0; u < 8; ++u) d[u] = *reinterpret_cast<const float4*>(q + 4 * u);
+                    __builtin_amdgcn_sched_barrier(0);  // the reads stay ahead of the adds
+                };
+                read(a, 0);
+                for (; c + 64 <= m; c += 64) {
+                    read(b, c + 32);
+#pragma unroll
+                    for (int u = 0; u < 8; ++u) fold(a[u]);
+                    read(a, c + 64);
+#pragma unroll
+                    for (int u = 0; u < 8; ++u) fold(b[u]);
+                }
+                if (c + 32 <= m) {
+#pragma unroll
+                    for (int u = 0; u < 8; ++u) fold(a[u]);
+                    c += 32;
+                }
+            }
+            for (; c + 4 <= m; c += 4) fold(*reinterpret_cast<const float4*>(t + c));
+            for (; c < m; ++c) acc = MAX ? fmaxf(acc, t[c]) : acc + t[c];
+        }
+    }
+    if (tid < rows && r0 + tid < nrows) y[r0 + tid] = acc;
+}
+
+// Outputs along a kept innermost axis, [outer][n][inner] -> [outer][inner], where there are too
+// few outputs for a thread each to keep memory busy: a workgroup takes 64 adjacent outputs, its
+// four wavefronts load every fourth element of the reduced axis, 16 deep, into LDS, and the first
+// wavefront folds the 64 elements of each output in order while the next 64 load.
+__global__ __launch_bounds__(256) void reduce_cols_kernel(const float* __restrict__ x,
+                                                          float* __restrict__ y, int kind,
+                                                          float init, int n, int inner,
+                                                          int blocks) {
+    __shared__ float tile[64 * 64];
+    constexpr int NL = 16;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int outer = blockIdx.x / blocks, i0 = (blockIdx.x - outer * blocks) * 64;
+    const bool ok = i0 + lane < inner;
+    const float* xp = x + (int64_t)outer * n * inner + i0 + (ok ? lane : 0);
+    float st[NL];
+    auto load = [&](int r0) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < NL; ++i) {
+            const int r = r0 + i * 4 + wave;
+            st[i] = ok && r < n ? xp[(int64_t)r * inner] : 0.0f;
+        }
+    };
+    load(0);
+    float acc = init;
+    for (int r0 = 0; r0 < n; r0 += 64) {
+        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < NL; ++i) tile[(i * 4 + wave) * 64 + lane] = st[i];
+        __syncthreads();
+        if (r0 + 64 < n) load(r0 + 64);
+        if (wave == 0) {
+            const int m = min(64, n - r0);
+#pragma unroll 8
+            for (int r = 0; r < m; ++r) {
+                const float v = tile[r * 64 + lane];
+                acc = kind ? fmaxf(acc, v) : acc + v;
+            }
+        }
+    }
+    if (wave == 0 && ok) y[(int64_t)outer * inner + i0 + lane] = acc;
 }
 
 // ---- hlo_strided_copy: push {r, total, dims[r], strides[r]}: out (row-major over dims) =
@@ -442,22 +602,62 @@ int launch_reduce_nd(const shp::Launch& l) {
     strides_of(sd, r, sst);
     p.rcount = 1;
     int64_t kept = 1;
+    // Axes in order, neighbours of one kind merged into one (sizes of 1 belong to either), which
+    // leaves the fold order and the output layout as they are.
+    int64_t outer = 1, inner = 1;  // kept elements before and after the reduced axes
+    int last = -1;                 // kind of the axis before: 1 reduced, 0 kept
     for (int k = 0; k < r; ++k) {
-        if (q[4 + r + k]) {
-            p.rdims[p.rr] = sd[k];
-            p.rstride[p.rr++] = sst[k];
-            p.rcount *= sd[k];
+        const int red = q[4 + r + k] ? 1 : 0;
+        if (!red) kept *= sd[k];
+        else p.rcount *= sd[k];
+        if (sd[k] == 1) continue;
+        int& cnt = red ? p.rr : p.rk;
+        int* dims = red ? p.rdims : p.kdims;
+        int64_t* st = red ? p.rstride : p.kstride;
+        if (last == red && (int64_t)dims[cnt - 1] * sd[k] < (1ll << 31)) {
+            dims[cnt - 1] *= sd[k];
         } else {
-            p.kdims[p.rk] = sd[k];
-            p.kstride[p.rk++] = sst[k];
-            kept *= sd[k];
+            dims[cnt] = sd[k];
+            ++cnt;
         }
+        st[cnt - 1] = sst[k];
+        if (!red) (p.rr ? inner : outer) *= sd[k];
+        last = red;
     }
     if (kept != q[2]) return shp::fail(SHP_ERR_SHAPE, "hlo_reduce: total != product of kept dims");
     rc = shp::check_total(l, q[2], "hlo_reduce");
     if (rc) return rc;
+    // One reduced run: rows of contiguous elements go through LDS tiles (the fewest rows per
+    // workgroup that still give every CU one).  So do columns up to 65,536 outputs, a wavefront
+    // per SIMD if each had a thread (7 x 300 x 800 over axis 1: 8 us against 60); with more
+    // outputs, and for other patterns, a thread per output keeps memory busy by itself.
+    const float* x = (const float*)l.in0;
+    float* y = (float*)l.out;
+    if (p.rr == 1 && p.rk <= 1 && inner == 1 && p.rcount >= 8) {
+        int rows = 256;
+        while (rows > 4 && (outer + rows - 1) / rows < 256) rows /= 2;
+        while (rows > 4 && rows * p.rcount >= (1ll << 28)) rows /= 2;  // 32-bit offsets
+        const int64_t wgs = (outer + rows - 1) / rows;
+        if (wgs < (1ll << 31) && rows * p.rcount < (1ll << 28)) {
+            const int n = (int)p.rcount;
+            const bool vec = n % 4 == 0 && ((uintptr_t)x & 15) == 0;
+            auto kern = p.kind ? (vec ? reduce_rows_kernel<true, true> : reduce_rows_kernel<false, true>)
+                               : (vec ? reduce_rows_kernel<true, false> : reduce_rows_kernel<false, false>);
+            hipLaunchKernelGGL(kern, dim3((unsigned)wgs), dim3(256), 0, l.stream, x, y, p.init, outer,
+                               n, rows);
+            SHP_HIP_CHECK(hipGetLastError());
+            return SHP_OK;
+        }
+    }
+    if (p.rr == 1 && inner > 1 && inner < (1 << 30) && p.rcount >= 16 && kept <= 65536) {
+        const int blocks = (int)((inner + 63) / 64);
+        hipLaunchKernelGGL(reduce_cols_kernel, dim3((unsigned)(outer * blocks)), dim3(256), 0,
+                           l.stream, x, y, p.kind, p.init, (int)p.rcount, (int)inner, blocks);
+        SHP_HIP_CHECK(hipGetLastError());
+        return SHP_OK;
+    }
     hipLaunchKernelGGL(reduce_nd_kernel, dim3(hlo_grid(l.out_elems)), dim3(kBlock), 0, l.stream,
-                       (const float*)l.in0, (float*)l.out, p, l.out_elems);
+                       x, y, p, l.out_elems);
     SHP_HIP_CHECK(hipGetLastError());
     return SHP_OK;
 }

@@ -956,7 +956,16 @@ def test_hlo_select(ctx, orc):
 
 
 @pytest.mark.parametrize("shape,dims", [((1, 4, 8, 64, 64), (4,)), ((1, 4, 8, 64, 64), (0, 2)),
-                                        ((3, 5, 7, 2, 3, 4), (1, 2, 5)), ((32, 7, 7, 2048), (1, 2))])
+                                        ((3, 5, 7, 2, 3, 4), (1, 2, 5)), ((32, 7, 7, 2048), (1, 2)),
+                                        # rows through LDS tiles: 4..256 rows a workgroup, one and
+                                        # several tiles, tails, unaligned rows, a single output
+                                        ((1024, 768), (1,)), ((1025, 767), (1,)), ((3, 2049), (1,)),
+                                        ((3, 8, 513), (1, 2)), ((70000, 33), (1,)), ((70001, 36), (1,)),
+                                        ((5000, 8), (1,)), ((5, 9000), (0, 1)), ((600, 7), (1,)),
+                                        # columns through LDS tiles and by thread, merged axes
+                                        ((2, 65, 130), (1,)), ((7, 27, 138), (0, 1)), ((1, 64, 1, 63), (1,)),
+                                        ((2, 16, 40000), (1,)), ((4, 130, 3, 1, 5), (1,)),
+                                        ((2, 40, 3, 50), (1, 3)), ((6, 1, 4), (1,))])
 def test_hlo_reduce(ctx, orc, shape, dims):
     """Sum folds in source order on both sides, so it is bit-exact like max."""
     from spirv_inference_amd import hlo_ops as H
