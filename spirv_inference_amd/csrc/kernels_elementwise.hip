@@ -12,6 +12,7 @@
 // handles 4 consecutive elements with 16-byte loads where the buffers allow it, in a
 // grid-stride loop sized for 256 CUs.
 #include "common.h"
+#include "runtime.h"
 
 namespace {
 
@@ -556,6 +557,40 @@ int launch_gather_rows(const shp::Launch& l) {
     return SHP_OK;
 }
 
+// ---- host staging (shp_run_kernel): pinned host memory to the bindings and back -----------
+// Bound by PCIe and by launch latency: one kernel moves both inputs (16 bytes a thread) and zeroes
+// the output, where three memsets and two copies each cost a submission.
+__device__ __forceinline__ void stage_copy(const float* __restrict__ s, float* __restrict__ d,
+                                           size_t n, size_t tid, size_t stride) {
+    const size_t n4 = n / 4;
+    for (size_t i = tid; i < n4; i += stride)
+        reinterpret_cast<ew4*>(d)[i] = reinterpret_cast<const ew4*>(s)[i];
+    for (size_t i = n4 * 4 + tid; i < n; i += stride) d[i] = s[i];
+}
+
+__global__ __launch_bounds__(kBlock) void host_stage_kernel(const float* __restrict__ p0,
+                                                            const float* __restrict__ p1, float* d0,
+                                                            size_t n0, float* d1, size_t n1,
+                                                            float* d2, size_t n2) {
+    const size_t tid = (size_t)blockIdx.x * kBlock + threadIdx.x;
+    const size_t stride = (size_t)gridDim.x * kBlock;
+    stage_copy(p0, d0, n0, tid, stride);
+    stage_copy(p1, d1, n1, tid, stride);
+    for (size_t i = tid; i < n2 / 4; i += stride)
+        reinterpret_cast<ew4*>(d2)[i] = ew4{0.f, 0.f, 0.f, 0.f};
+    for (size_t i = n2 / 4 * 4 + tid; i < n2; i += stride) d2[i] = 0.0f;
+    if (tid == 0) {  // an unused binding holds one zero
+        if (!n0) d0[0] = 0.0f;
+        if (!n1) d1[0] = 0.0f;
+        if (!n2) d2[0] = 0.0f;
+    }
+}
+
+__global__ __launch_bounds__(kBlock) void host_fetch_kernel(const float* __restrict__ d,
+                                                            float* __restrict__ p, size_t n) {
+    stage_copy(d, p, n, (size_t)blockIdx.x * kBlock + threadIdx.x, (size_t)gridDim.x * kBlock);
+}
+
 // ---- counter-based RNG fill ----------------------------------------------------------
 __device__ __forceinline__ uint64_t mix64(uint64_t z) {
     z += 0x9E3779B97F4A7C15ull;
@@ -589,6 +624,21 @@ __global__ __launch_bounds__(kBlock) void fill_random_kernel(float* __restrict__
 }  // namespace
 
 namespace shp {
+
+int host_stage_launch(hipStream_t s, const float* p0, const float* p1, float* d0, size_t n0,
+                      float* d1, size_t n1, float* d2, size_t n2) {
+    const size_t most = std::max(std::max(n0, n1), n2);
+    hipLaunchKernelGGL(host_stage_kernel, dim3(ew_grid(most / 4 + 1)), dim3(kBlock), 0, s, p0, p1,
+                       d0, n0, d1, n1, d2, n2);
+    SHP_HIP_CHECK(hipGetLastError());
+    return SHP_OK;
+}
+
+int host_fetch_launch(hipStream_t s, const float* d2, float* p, size_t n2) {
+    hipLaunchKernelGGL(host_fetch_kernel, dim3(ew_grid(n2 / 4 + 1)), dim3(kBlock), 0, s, d2, p, n2);
+    SHP_HIP_CHECK(hipGetLastError());
+    return SHP_OK;
+}
 
 int fill_random(hipStream_t stream, float* p, uint64_t n, uint64_t seed, uint64_t tensor_id,
                 int kind, float lo, float hi) {

@@ -424,7 +424,7 @@ __global__ __launch_bounds__(kBlock) void reduce_nd_kernel(const float* __restri
 // loads into registers and then LDS (rows padded by 4 floats, so 16-byte reads down a column of
 // rows are free of bank conflicts), while the tile before it is folded by the first `rows`
 // threads.  Few rows per workgroup when there are few rows at all: 1,024 rows of 768 take four
-// each, one per CU, 114 us with a thread walking each row and 7.1 us so (10.5 before the LDS reads
+// each, one per CU: 114 us with a thread walking each row, 5.4 us so (10.5 before the LDS reads
 // were kept a batch ahead of the adds).
 constexpr int kRedTile = 8192;
 
@@ -629,7 +629,7 @@ int launch_reduce_nd(const shp::Launch& l) {
     if (rc) return rc;
     // One reduced run: rows of contiguous elements go through LDS tiles (the fewest rows per
     // workgroup that still give every CU one).  So do columns up to 65,536 outputs, a wavefront
-    // per SIMD if each had a thread (7 x 300 x 800 over axis 1: 8 us against 60); with more
+    // per SIMD if each had a thread (7 x 300 x 800 over axis 1: 8.4 us against 48); with more
     // outputs, and for other patterns, a thread per output keeps memory busy by itself.
     const float* x = (const float*)l.in0;
     float* y = (float*)l.out;

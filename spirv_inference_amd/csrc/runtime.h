@@ -24,6 +24,18 @@ struct Ctx {
     std::vector<float*> retired;
     GemmTune tune;  // planner overrides of this context's dense launches (shp_tune)
 
+    // Device buffers and staging memory of shp_run_kernel, kept from call to call (a call is
+    // synchronous, so none is in use between calls): three bindings of up to kIoKeep bytes, and
+    // kIoStage bytes of pinned memory in each direction.
+    static constexpr size_t kIoKeep = 64u << 20, kIoStage = 1u << 20;
+    void* io[3] = {nullptr, nullptr, nullptr};
+    size_t io_bytes[3] = {0, 0, 0};
+    char *stage_up = nullptr, *stage_down = nullptr;
+    hipEvent_t io_events[2] = {nullptr, nullptr};
+    bool io_used = false;
+    int io_prepare();                          // events; pinned memory from the second call on
+    int io_buffer(int i, size_t bytes);        // binding i of at least this size
+
     struct Timer {
         hipEvent_t a, b;
         std::string name;
@@ -48,6 +60,12 @@ struct Ctx {
 // call made between shp_capture_begin and shp_capture_end fails closed instead of recording
 // a memset or copy node into the caller's graph or breaking the capture.
 int refuse_while_capturing(hipStream_t stream, const char* what);
+
+// shp_run_kernel's bindings, uploaded from pinned memory (both device-visible; n0 or n1 may be 0)
+// with the output zeroed, and the output downloaded to it: one kernel each way.
+int host_stage_launch(hipStream_t s, const float* pinned0, const float* pinned1, float* d0,
+                      size_t n0, float* d1, size_t n1, float* d2, size_t n2);
+int host_fetch_launch(hipStream_t s, const float* d2, float* pinned, size_t n2);
 
 // Resolves, once per device and with that device current, the device address of the fixed
 // split-K scratch array behind shp_launch_static (static_scratch.hip).

@@ -164,7 +164,7 @@ class Context:
         """Synchronous host-to-host call with the semantics of vulkan.rs:42-44."""
         a0 = np.ascontiguousarray(spec.input0, dtype=np.float32).reshape(-1)
         a1 = np.ascontiguousarray(spec.input1, dtype=np.float32).reshape(-1)
-        out = np.zeros(spec.output_elements, dtype=np.float32)
+        out = np.empty(spec.output_elements, dtype=np.float32)
         arr, n = _push(spec.push)
         info = RunInfo()
         rc = lib().shp_run_kernel(self.handle, spec.kernel.encode(), a0.ctypes.data, a0.size,

@@ -985,6 +985,37 @@ def test_hlo_shape_ops_fail_closed(ctx):
         _dev(ctx, "hlo_slice", rnd(4, 6), None, 5, H.slice_push((4, 6), (0, 0), (2, 6)))
 
 
+@pytest.mark.parametrize("n", [1, 3, 1000, 131073, 262143, 262144, 262145, 300001, (16 << 20) + 5])
+def test_run_kernel_sizes(n):
+    """Host buffers in and out around the pinned-staging (1 MiB each way) and kept-buffer (64 MiB)
+    limits, a first and later calls of one context, larger and smaller than the call before."""
+    from spirv_inference_amd import Context, KernelRun
+    none = np.zeros(1, np.float32)
+    with Context("any") as c:
+        for m in (n, n, max(1, n // 2), n):
+            x, y = rnd(m), rnd(m)
+            got = c.run_kernel(KernelRun("add", "add", x, y, m, 1, [m])).values
+            np.testing.assert_array_equal(got, x + y)
+            out = c.run_kernel(KernelRun("relu", "relu", x, none, m, 1, [m]))
+            np.testing.assert_array_equal(out.values, np.maximum(x, 0))
+            assert out.elapsed_ms > 0
+
+
+def test_run_kernel_output_starts_at_zero(ctx):
+    """A kernel that writes part of its output leaves zeros in the rest, whatever ran before."""
+    from spirv_inference_amd import KernelRun
+    from spirv_inference_amd import hlo_ops as H
+    none = np.zeros(0, np.float32)
+    for n in (40, 400000):
+        ctx.run_kernel(KernelRun("fill", "relu", np.ones(4 * n, np.float32), none, 4 * n, 1, [4 * n]))
+        x = rnd(2, n)
+        got = ctx.run_kernel(KernelRun("c", "hlo_concatenate_into", x, none, 4 * n, 1,
+                                       H.concatenate_into_push((2, 2 * n), (2, n), 1, n))).values
+        want = np.zeros((2, 2 * n), np.float32)
+        want[:, n:] = x
+        np.testing.assert_array_equal(got.reshape(2, 2 * n), want)
+
+
 @pytest.mark.parametrize("n,nan_at", [(0, []), (7, []), (7, [3]), (4099, [4098, 17, 2000]),
                                       (1 << 22, [(1 << 22) - 1, 123457, 1 << 21])])
 def test_nan_count(ctx, orc, n, nan_at):
