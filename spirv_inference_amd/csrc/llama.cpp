@@ -463,7 +463,10 @@ int shp_llama_create(shp_ctx* ctx, const shp_llama_config* cfg, uint64_t seed, s
     if (!rc) rc = lm->setup_prefill();
     if (!rc && lm->p_grid > 0) lm->engine = SHP_LLAMA_PERSISTENT;
     if (!rc) {
+        // the fills on the context's stream and the clears on the null stream, which the
+        // context's stream does not wait for
         hipError_t e = hipStreamSynchronize(lm->ctx->stream);
+        if (e == hipSuccess) e = hipStreamSynchronize(nullptr);
         if (e != hipSuccess) rc = fail(SHP_ERR_HIP, hipGetErrorString(e));
     }
     if (rc) {

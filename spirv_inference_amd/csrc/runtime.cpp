@@ -120,6 +120,9 @@ int Ctx::ensure_workspace(size_t bytes) {
     workspace_bytes = bytes;
     // the split-K tile counters at its start must begin at zero (launches keep them zero)
     SHP_HIP_CHECK(hipMemset(workspace, 0, std::min(bytes, kSplitCounterBytes)));
+    // hipMemset does not wait on the host, and the context's stream does not wait for the null
+    // stream: without this the first launches could count on counters not yet cleared
+    SHP_HIP_CHECK(hipStreamSynchronize(nullptr));
     return SHP_OK;
 }
 
