@@ -53,6 +53,9 @@ struct GemmTune {
     // fully_connected with 2-16 rows: the split-K MFMA kernel where it takes the shape (0) or
     // the wavefront-per-column and tiled kernels (-1)
     int fc = 0;
+    // products and convolutions on gemm_direct_kernel where it is expected to win (0), wherever it
+    // takes the operands with k K-splits (k > 0), never (-1)
+    int direct = 0;
 };
 
 // Everything a launcher needs: the three bindings, the push vector and the epilogue.

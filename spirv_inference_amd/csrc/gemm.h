@@ -51,8 +51,8 @@ struct GemmParams {
     // tile order: bands of group_m tile rows, each band walked column by column (1: row
     // major); each XCD then takes a contiguous run of that order (tile_coords)
     int group_m;
-    // 1: [rows] x [out][in]^T products with MFMA chains of at most 64 k where gemm_bl_kernel
-    // takes them (64x64 tiles only); see there
+    // 1: [rows] x [out][in]^T products with MFMA chains of at most 32 k where gemm_bl_kernel
+    // takes them (64x64 tiles, K tiles to 32); see there
     int short_chains;
 };
 
@@ -70,5 +70,13 @@ int gemm_launch(hipStream_t stream, GemmParams p, int amode, int bmode, int cmod
 // Workspace the launcher would like for this problem (0 if it will not split K).
 size_t gemm_workspace_bytes(const GemmParams& p, int amode, int bmode, int cmode,
                             const GemmTune* tune);
+
+// The small-problem kernel (kernels_gemm_direct.hip): whether it takes the operands at all, with
+// how many K splits it should run (0: the tiled kernels are better), its workspace, its launch.
+bool direct_eligible(const GemmParams& p, int amode, int bmode, int cmode);
+int direct_splits(const GemmParams& p, int tune);
+size_t direct_workspace(const GemmParams& p, int splits);
+int direct_launch(hipStream_t stream, GemmParams p, int amode, int bmode, int splits,
+                  float* workspace);
 
 }  // namespace shp

@@ -636,9 +636,9 @@ __device__ __host__ inline int64_t bl_b_extent(const GemmParams& p, int bmode) {
 }
 
 //
-// FL cuts the MFMA chains every 64 k (32 with the 16-deep tile) and adds them to a second
-// accumulator set, for callers whose sums must not lose to a vector-unit reduction (the decoder's
-// prompt pass against its token steps): 3 % more issue slots.
+// FL cuts the MFMA chains after every K tile and adds them to one of two further accumulator sets
+// in turn, for callers whose sums must not lose to a vector-unit reduction (the decoder's prompt
+// pass against its token steps): 3 % more issue slots.
 template <int BM, int BN, int BK, int AM, int BMD, bool FL = false>
 __global__ __launch_bounds__(256) void gemm_bl_kernel(GemmParams p) {
     static_assert(AM == shp::A_KVEC || AM == shp::A_CONV_NHWC4, "row-contiguous A");
@@ -753,7 +753,7 @@ __global__ __launch_bounds__(256) void gemm_bl_kernel(GemmParams p) {
         }
     };
 
-    floatx16 acc[FM][FN], sum[FL ? FM : 1][FL ? FN : 1];
+    floatx16 acc[FM][FN], sum[2][FL ? FM : 1][FL ? FN : 1];
 #pragma unroll
     for (int i = 0; i < FM; ++i)
 #pragma unroll
@@ -761,9 +761,9 @@ __global__ __launch_bounds__(256) void gemm_bl_kernel(GemmParams p) {
 #pragma unroll
             for (int r = 0; r < 16; ++r) {
                 acc[i][j][r] = 0.0f;
-                if constexpr (FL) sum[i][j][r] = 0.0f;
+                if constexpr (FL) sum[0][i][j][r] = sum[1][i][j][r] = 0.0f;
             }
-    auto flush = [&]() __attribute__((always_inline)) {
+    auto flush = [&](int par) __attribute__((always_inline)) {
         if constexpr (FL) {
 #pragma unroll
             for (int i = 0; i < FM; ++i)
@@ -771,7 +771,7 @@ __global__ __launch_bounds__(256) void gemm_bl_kernel(GemmParams p) {
                 for (int j = 0; j < FN; ++j)
 #pragma unroll
                     for (int r = 0; r < 16; ++r) {
-                        sum[i][j][r] += acc[i][j][r];
+                        sum[par][i][j][r] += acc[i][j][r];
                         acc[i][j][r] = 0.0f;
                     }
         }
@@ -848,15 +848,15 @@ __global__ __launch_bounds__(256) void gemm_bl_kernel(GemmParams p) {
         int kt = 0;
         for (; kt + 1 < ntk; kt += 2) {
             tile(0, s1, true, s0, min(kt + 2, ntk - 1));
-            if constexpr (BK == 64) flush();
+            flush(0);
             __syncthreads();
             tile(1, s0, kt + 2 < ntk, s1, min(kt + 3, ntk - 1));
-            flush();
+            flush(1);
             __syncthreads();
         }
         if (kt < ntk) {
             tile(0, s1, false, s0, kt);
-            flush();
+            flush(0);
             __syncthreads();
         }
     }
@@ -864,7 +864,7 @@ __global__ __launch_bounds__(256) void gemm_bl_kernel(GemmParams p) {
 #pragma unroll
         for (int i = 0; i < FM; ++i)
 #pragma unroll
-            for (int j = 0; j < FN; ++j) acc[i][j] = sum[i][j];
+            for (int j = 0; j < FN; ++j) acc[i][j] = sum[0][i][j] + sum[1][i][j];
 
     gemm_epilogue<BM, BN, 2, 2, RC, CS, shp::C_STRIDED>(p, acc, smem, m0, n0, split, p.splits, bz,
                                                         bo, bi, gridDim.z,
@@ -2017,10 +2017,8 @@ int bl_mask(const GemmParams& p, int am, int bm, int cm) {
 template <int AM, int BMD>
 void launch_bl_combo(hipStream_t s, const GemmParams& p, TileCfg t, dim3 grid) {
     if constexpr (AM == shp::A_KVEC && BMD == shp::B_KVEC) {
-        if (p.short_chains && t.bm == 64) {
-            if (t.bk == 64)
-                hipLaunchKernelGGL((gemm_bl_kernel<64, 64, 64, AM, BMD, true>), grid, dim3(256), 0, s, p);
-            else if (t.bk == 16)
+        if (p.short_chains && t.bm == 64 && t.bk <= 32) {
+            if (t.bk == 16)
                 hipLaunchKernelGGL((gemm_bl_kernel<64, 64, 16, AM, BMD, true>), grid, dim3(256), 0, s, p);
             else
                 hipLaunchKernelGGL((gemm_bl_kernel<64, 64, 32, AM, BMD, true>), grid, dim3(256), 0, s, p);
@@ -2276,7 +2274,7 @@ bool plan_bl(const GemmParams& p, int nbatch, int blm, const shp::GemmTune& tn, 
         const int ti = t.bm == 128 ? (t.bn == 128 ? 1 : 2) : 3;
         if (tn.tile && tn.tile != ti) continue;
         if (tn.bk && tn.bk != t.bk) continue;
-        if (p.short_chains && t.bm == 128) continue;
+        if (p.short_chains && (t.bm == 128 || t.bk == 64)) continue;
         const int kq = t.bk == 64 ? 64 : 32;
         for (int s : kSplits) {
             if (tn.splits && tn.splits != s) continue;
@@ -2349,6 +2347,13 @@ int dot_modes(const GemmParams& p, int& am, int& bm);
 
 namespace shp {
 
+// A forced tile, K tile, split count or kernel keeps the tiled kernels, unless the direct kernel is
+// forced itself.
+static int direct_tune(const GemmTune& t) {
+    if (t.direct) return t.direct;
+    return t.tile || t.bk || t.splits || t.dma || t.pg || t.bl || t.table < 0 ? -1 : 0;
+}
+
 size_t gemm_workspace_bytes(const GemmParams& p, int amode, int bmode, int cmode,
                             const GemmTune* tune) {
     static const GemmTune kAuto;
@@ -2364,8 +2369,11 @@ size_t gemm_workspace_bytes(const GemmParams& p, int amode, int bmode, int cmode
                             amode, bmode, b);
         splits = std::max(splits, pl.splits);
     }
-    if (splits <= 1) return 0;
-    return kSplitCounterBytes + (size_t)splits * nbatch * p.M * p.N * sizeof(float);
+    size_t direct = 0;
+    if (direct_eligible(p, amode, bmode, cmode))
+        direct = direct_workspace(p, direct_splits(p, tune ? direct_tune(*tune) : 0));
+    if (splits <= 1) return direct;
+    return std::max(direct, kSplitCounterBytes + (size_t)splits * nbatch * p.M * p.N * sizeof(float));
 }
 
 size_t gemm_workspace_for_kernel(const char* name, const int32_t* q, size_t n,
@@ -2416,6 +2424,8 @@ size_t gemm_workspace_for_kernel(const char* name, const int32_t* q, size_t n,
         return 0;
     }
     if (p.M <= 0 || p.N <= 0 || p.K <= 0) return 0;
+    p.scm = p.N;  // the row stride of every form but dot_general_strided's, which only the direct
+    p.scn = 1;    // kernel's eligibility reads
     size_t small_ws = 0;  // the K-split small-product path of a 1x1 conv2d_nhwc
     if (k == "conv2d_nhwc" && q[7] == 1 && q[8] == 1 && q[9] == 1 && q[10] == 1 &&
         q[12] == 0 && q[13] == 0 && q[5] == q[2] && q[6] == q[3])
@@ -2500,6 +2510,11 @@ int gemm_launch(hipStream_t stream, GemmParams p, int amode, int bmode, int cmod
     if (tn.sk >= 0) {
         const int v = smallk_variant(p, amode, bmode, cmode, nbatch);
         if (v) return launch_smallk(stream, p, amode, v);
+    }
+    if (direct_eligible(p, amode, bmode, cmode)) {
+        const int ds = direct_splits(p, direct_tune(tn));
+        if (ds == 1 || (ds > 1 && workspace && workspace_bytes >= direct_workspace(p, ds)))
+            return direct_launch(stream, p, amode, bmode, ds, workspace);
     }
     const int blm = bl_mask(p, amode, bmode, cmode);
     Plan pl = plan_gemm(p, nbatch, hot, dma_ok, amode == A_CONV_NHWC4, tn, amode, bmode, blm);

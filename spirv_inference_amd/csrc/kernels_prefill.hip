@@ -4,8 +4,8 @@
 // Feeding a prompt token by token reads all 4.1 GB of TinyLlama's weights per position
 // (0.76 ms each); a chunk of positions reads them once.  Up to 64 rows the products are bound by
 // that read, so they have their own kernel (skinny_kernel); above, they are matrix-core bound and
-// run on the tiled GEMM kernels.  TinyLlama's shape, whole prompt: 32 ids 24.3 -> 2.45 ms,
-// 384 ids 291 -> 8.6 ms; 1.8 ms is the least (2 ids, two token steps took 1.5).
+// run on the tiled GEMM kernels.  TinyLlama's shape, whole prompt: 32 ids 24.3 -> 2.26 ms,
+// 384 ids 291 -> 9.1 ms; 1.6 ms is the least (2 ids, two token steps take 1.5).
 #include "prefill.h"
 #include "coherent.h"
 
@@ -27,32 +27,37 @@ __device__ __forceinline__ floatx4 mfma4(f4v a, f4v b, floatx4 c) {
 }
 
 // ---- skinny_kernel: out = x[M][K] w[N][K]^T for M <= 16 MT rows -------------------------------
-// HBM bound: 4 N K bytes of weights, each read once.  A workgroup of four wavefronts takes 32
-// weight rows over one K range; the wavefronts take 128-byte pieces of the rows in turn (so a
-// workgroup reads 512 contiguous bytes of each row per step) straight into the MFMA operand
-// layout, no LDS and no barrier in the loop: lane l loads 16 bytes of row l % 16, k + 4 * (l / 16).
-// The x rows are read the same way and come from L2 (256 KB at 32 rows of 2,048).  Two register
-// sets alternate, so a wavefront has up to 8 KB of weights in flight.  The MFMA chains are cut
-// every 64 k and added to a second accumulator: the sum's rounding error is then that of the
-// decode step's GEMV (lanes of ~32 terms and a tree), where one chain over K had 1.6 times it.
-// The four partial tiles are summed in LDS in wavefront order.  D = w x^T puts four consecutive n of one row m in a lane:
-// 16-byte stores, and gate and up of one output next to each other for the SwiGLU form.
+// HBM bound: 4 N K bytes of weights, each read once, so what counts is bytes in flight.  A
+// workgroup of eight wavefronts takes 32 weight rows over one K range (gridDim.y of them); each
+// wavefront takes an eighth of the range and loads its 16-deep steps straight into the MFMA operand
+// layout, no LDS and no barrier in the loop: lane l loads 16 bytes of row l % 16 at k + 4 * (l / 16).
+// The x rows are read the same way and come from L2 (256 KB at 32 rows of 2,048).  Four steps ahead
+// of the products, so a wavefront has 8 KB of weights in flight and a CU about 100 (TinyLlama at 32
+// rows: gate/up 41 us for 92 MB, the others 13 us; a form with x stationary in registers and 128 KB in
+// flight took 34 and 19, loading x into every CU first costs the small ones more).  The eight partial
+// tiles are summed in LDS in wavefront order.  The MFMA chains are cut every 32 k and added to a
+// second accumulator: the sum's rounding error is then that of the decode step's GEMV (lanes of ~32
+// terms and a tree), where one chain had 1.6 times it.  D = w x^T puts four consecutive n of one row
+// m in a lane: 16-byte stores, and gate and up of one output next to each other for the SwiGLU form.
 constexpr unsigned kOob = 0x80000000u;  // past every operand range: loads return 0
+constexpr int kSkWaves = 8;
 
 template <int MT, int MODE>
-__global__ __launch_bounds__(256) void skinny_kernel(const float* __restrict__ x,
-                                                     const float* __restrict__ w,
-                                                     float* __restrict__ out, int M, int N, int K,
-                                                     int kper) {
-    constexpr int NT = 2, WV = 4, STEP = 32 * WV;
-    __shared__ __attribute__((aligned(16))) f4v red[MT * NT][WV][64];
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+__global__ __launch_bounds__(kSkWaves * 64, MT <= 2 ? 4 : 2) void skinny_kernel(
+    const float* __restrict__ x, const float* __restrict__ w, float* __restrict__ out, int M, int N,
+    int K, int kper) {
+    constexpr int NT = 2, ST = 5;
+    __shared__ __attribute__((aligned(16))) f4v red[MT * NT][kSkWaves][64];
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int g = lane >> 4, li = lane & 15;
     const int n0 = blockIdx.x * 32;
     const int kb = blockIdx.y * kper, ke = min(K, kb + kper);
+    const int steps = max(0, (ke - kb + 15) >> 4);
+    const int s0 = steps * wave / kSkWaves, ns = steps * (wave + 1) / kSkWaves - s0;
+    const int k0 = kb + 16 * s0 + 4 * g;
     const __amdgpu_buffer_rsrc_t wr = buffer_rsrc(w, (int64_t)N * K);
     const __amdgpu_buffer_rsrc_t xr = buffer_rsrc(x, (int64_t)M * K);
-    const int k0 = kb + wave * 32 + 4 * g;
     unsigned wo[NT], xo[MT];
 #pragma unroll
     for (int i = 0; i < NT; ++i) {
@@ -64,21 +69,21 @@ __global__ __launch_bounds__(256) void skinny_kernel(const float* __restrict__ x
         const int m = 16 * i + li;
         xo[i] = m < M ? (unsigned)(((int64_t)m * K + k0) * 4) : kOob;
     }
-    struct Set { f4v w[2][NT], x[2][MT]; };
-    auto load = [&](int it, Set& s) __attribute__((always_inline)) {
-        const unsigned so = (unsigned)(it * STEP * 4);
+    struct Set { f4v w[NT], x[MT]; };
+    Set st[ST];
+    auto load = [&](int s, Set& d) __attribute__((always_inline)) {
+        // K % 4 == 0, so a lane's 16 bytes lie on one side of the end; past it (also the steps
+        // beyond ns) nothing is read
+        const bool in = s < ns && k0 + 16 * s < ke;
+        const unsigned so = (unsigned)(s * 64);
 #pragma unroll
-        for (int u = 0; u < 2; ++u) {
-            const bool in = k0 + it * STEP + 16 * u < ke;
+        for (int i = 0; i < NT; ++i)
+            d.w[i] = __builtin_bit_cast(
+                f4v, __builtin_amdgcn_raw_buffer_load_b128(wr, in ? wo[i] : kOob, so, 0));
 #pragma unroll
-            for (int i = 0; i < NT; ++i)
-                s.w[u][i] = __builtin_bit_cast(f4v, __builtin_amdgcn_raw_buffer_load_b128(
-                    wr, in ? wo[i] + 64u * u : kOob, so, 0));
-#pragma unroll
-            for (int i = 0; i < MT; ++i)
-                s.x[u][i] = __builtin_bit_cast(f4v, __builtin_amdgcn_raw_buffer_load_b128(
-                    xr, in ? xo[i] + 64u * u : kOob, so, 0));
-        }
+        for (int i = 0; i < MT; ++i)
+            d.x[i] = __builtin_bit_cast(
+                f4v, __builtin_amdgcn_raw_buffer_load_b128(xr, in ? xo[i] : kOob, so, 0));
     };
     floatx4 acc[MT][NT], sum[MT][NT];
     const floatx4 zero = {0.f, 0.f, 0.f, 0.f};
@@ -86,38 +91,33 @@ __global__ __launch_bounds__(256) void skinny_kernel(const float* __restrict__ x
     for (int i = 0; i < MT; ++i)
 #pragma unroll
         for (int j = 0; j < NT; ++j) acc[i][j] = sum[i][j] = zero;
-    auto flush = [&]() __attribute__((always_inline)) {
+    auto mul = [&](const Set& s, bool cut) __attribute__((always_inline)) {
 #pragma unroll
         for (int i = 0; i < MT; ++i)
 #pragma unroll
             for (int j = 0; j < NT; ++j) {
-                sum[i][j] += acc[i][j];
-                acc[i][j] = zero;
+                acc[i][j] = mfma4(s.w[j], s.x[i], acc[i][j]);
+                if (cut) {
+                    sum[i][j] += acc[i][j];
+                    acc[i][j] = zero;
+                }
             }
     };
-    auto mul = [&](const Set& s) __attribute__((always_inline)) {
 #pragma unroll
-        for (int u = 0; u < 2; ++u)
+    for (int u = 0; u < ST - 1; ++u) load(u, st[u]);
+    int s = 0;
+    for (; s + ST <= ns; s += ST) {
 #pragma unroll
-            for (int i = 0; i < MT; ++i)
-#pragma unroll
-                for (int j = 0; j < NT; ++j) acc[i][j] = mfma4(s.w[u][j], s.x[u][i], acc[i][j]);
-    };
-    const int nit = (ke - kb + STEP - 1) / STEP;
-    Set a, b;
-    load(0, a);
-    int it = 0;
-    for (; it + 1 < nit; it += 2) {
-        load(it + 1, b);
-        mul(a);
-        if (it + 2 < nit) load(it + 2, a);
-        mul(b);
-        flush();
+        for (int u = 0; u < ST; ++u) {
+            load(s + u + ST - 1, st[(u + ST - 1) % ST]);
+            __builtin_amdgcn_sched_barrier(0);  // the loads stay ahead of the products
+            mul(st[u], (u & 1) || u == ST - 1);
+            __builtin_amdgcn_sched_barrier(0);
+        }
     }
-    if (it < nit) {
-        mul(a);
-        flush();
-    }
+#pragma unroll
+    for (int u = 0; u < ST - 1; ++u)
+        if (s + u < ns) mul(st[u], true);
 
 #pragma unroll
     for (int i = 0; i < MT; ++i)
@@ -125,20 +125,20 @@ __global__ __launch_bounds__(256) void skinny_kernel(const float* __restrict__ x
         for (int j = 0; j < NT; ++j)
             red[i * NT + j][wave][lane] = f4v{sum[i][j][0], sum[i][j][1], sum[i][j][2], sum[i][j][3]};
     __syncthreads();
-    for (int t = wave; t < MT * NT; t += WV) {
-        f4v v = red[t][0][lane];
+    const int t = wave;
+    if (t >= MT * NT) return;
+    f4v v = red[t][0][lane];
 #pragma unroll
-        for (int u = 1; u < WV; ++u) v += red[t][u][lane];
-        const int m = 16 * (t / NT) + li, n = n0 + 16 * (t % NT) + 4 * g;
-        if (m >= M || n >= N) continue;
-        if constexpr (MODE == shp::SK_SWIGLU) {
-            float2 r;
-            r.x = (v.x * (1.0f / (1.0f + expf(-v.x)))) * v.y;
-            r.y = (v.z * (1.0f / (1.0f + expf(-v.z)))) * v.w;
-            *reinterpret_cast<float2*>(out + ((int64_t)m * N + n) / 2) = r;
-        } else {
-            *reinterpret_cast<f4v*>(out + ((int64_t)blockIdx.y * M + m) * N + n) = v;
-        }
+    for (int u = 1; u < kSkWaves; ++u) v += red[t][u][lane];
+    const int m = 16 * (t / NT) + li, n = n0 + 16 * (t % NT) + 4 * g;
+    if (m >= M || n >= N) return;
+    if constexpr (MODE == shp::SK_SWIGLU) {
+        float2 r;
+        r.x = (v.x * (1.0f / (1.0f + expf(-v.x)))) * v.y;
+        r.y = (v.z * (1.0f / (1.0f + expf(-v.z)))) * v.w;
+        *reinterpret_cast<float2*>(out + ((int64_t)m * N + n) / 2) = r;
+    } else {
+        *reinterpret_cast<f4v*>(out + ((int64_t)blockIdx.y * M + m) * N + n) = v;
     }
 }
 
@@ -166,10 +166,15 @@ __global__ __launch_bounds__(256) void prefill_norm_kernel(const float* x,
     for (int i = threadIdx.x; i < h4; i += 256) {
         f4v v = xr[i];
         if (splits) {
-            f4v t = {0.f, 0.f, 0.f, 0.f};
-            for (int s = 0; s < splits; ++s)
-                t += *(reinterpret_cast<const f4v*>(part + s * sstride) + base + i);
-            v += t;
+            f4v t[shp::kSkinnySplits];  // every partial in flight before the first is added
+#pragma unroll
+            for (int s = 0; s < shp::kSkinnySplits; ++s)
+                if (s < splits) t[s] = *(reinterpret_cast<const f4v*>(part + s * sstride) + base + i);
+            f4v sum = t[0];
+#pragma unroll
+            for (int s = 1; s < shp::kSkinnySplits; ++s)
+                if (s < splits) sum += t[s];
+            v += sum;
             xo[i] = v;
         }
         ss += v.x * v.x + v.y * v.y + v.z * v.z + v.w * v.w;
@@ -196,11 +201,20 @@ __global__ __launch_bounds__(256) void prefill_rope_kernel(const float* __restri
     const int e = blockIdx.y * 256 + threadIdx.x, hd = e >> 5, j = e & 31;
     if (hd >= heads) return;
     const int64_t o = (int64_t)row * heads * 64 + hd * 64 + j;
-    float a = 0.0f, b = 0.0f;
-    for (int s = 0; s < splits; ++s) {
-        a += part[s * sstride + o];
-        b += part[s * sstride + o + 32];
-    }
+    float ta[shp::kSkinnySplits], tb[shp::kSkinnySplits];
+#pragma unroll
+    for (int s = 0; s < shp::kSkinnySplits; ++s)
+        if (s < splits) {
+            ta[s] = part[s * sstride + o];
+            tb[s] = part[s * sstride + o + 32];
+        }
+    float a = ta[0], b = tb[0];
+#pragma unroll
+    for (int s = 1; s < shp::kSkinnySplits; ++s)
+        if (s < splits) {
+            a += ta[s];
+            b += tb[s];
+        }
     const int pos = pos0 + row;
     if (hd >= n_heads + n_kv) {
         float* d = vc + ((int64_t)(hd - n_heads - n_kv) * max_seq + pos) * 64 + j;
@@ -272,12 +286,12 @@ __global__ __launch_bounds__(1024) void prefill_argmax_kernel(const float* __res
 
 namespace shp {
 
+// Splits grow while every CU still gets at most about one workgroup and a wavefront keeps two
+// steps (TinyLlama: QKV 80 row groups x 3, Wo 64 x 4, down 64 x 4; gate/up's 352 need none).
 int skinny_splits(int N, int K) {
-    // Enough workgroups for two or three per CU (each holds up to 32 KB of weights in flight),
-    // but at least one 128-deep step per wavefront set.
-    const int groups = (N + 31) / 32, steps = (K + 127) / 128;
+    const int groups = (N + 31) / 32, steps = (K + 15) / 16;
     int s = 1;
-    while (s < kSkinnySplits && groups * s < 512 && s * 2 <= steps) s *= 2;
+    while (s < kSkinnySplits && groups * (s + 1) <= 256 && steps / (s + 1) >= 2 * kSkWaves) ++s;
     return s;
 }
 
@@ -286,21 +300,15 @@ int skinny_launch(hipStream_t st, const float* x, int M, const float* w, int N, 
     if (M <= 0 || M > kSkinnyRows || N <= 0 || N % 8 || K <= 0 || K % 4 || splits < 1 ||
         (mode == SK_SWIGLU && splits != 1) || (int64_t)N * K * 4 >= (1ll << 31))
         return fail(SHP_ERR_SHAPE, "skinny product: shape");
-    const int kper = (((K + splits - 1) / splits) + 127) / 128 * 128;
-    const dim3 grid((unsigned)((N + 31) / 32), (unsigned)splits);
+    const int kper = ((K + 15) / 16 + splits - 1) / splits * 16;
+    const dim3 grid((unsigned)((N + 31) / 32), (unsigned)splits), block(kSkWaves * 64);
     const int mt = (M + 15) / 16;
-#define SHP_SKINNY(MT)                                                                        \
-    if (mode == SK_SWIGLU)                                                                    \
-        hipLaunchKernelGGL((skinny_kernel<MT, SK_SWIGLU>), grid, dim3(256), 0, st, x, w, out, \
-                           M, N, K, kper);                                                    \
-    else                                                                                      \
-        hipLaunchKernelGGL((skinny_kernel<MT, SK_PARTIAL>), grid, dim3(256), 0, st, x, w, out, \
-                           M, N, K, kper);
-    if (mt == 1) { SHP_SKINNY(1) }
-    else if (mt == 2) { SHP_SKINNY(2) }
-    else if (mt == 3) { SHP_SKINNY(3) }
-    else { SHP_SKINNY(4) }
-#undef SHP_SKINNY
+    const bool sw = mode == SK_SWIGLU;
+    auto kern = mt == 1   ? (sw ? skinny_kernel<1, SK_SWIGLU> : skinny_kernel<1, SK_PARTIAL>)
+                : mt == 2 ? (sw ? skinny_kernel<2, SK_SWIGLU> : skinny_kernel<2, SK_PARTIAL>)
+                : mt == 3 ? (sw ? skinny_kernel<3, SK_SWIGLU> : skinny_kernel<3, SK_PARTIAL>)
+                          : (sw ? skinny_kernel<4, SK_SWIGLU> : skinny_kernel<4, SK_PARTIAL>);
+    hipLaunchKernelGGL(kern, grid, block, 0, st, x, w, out, M, N, K, kper);
     SHP_HIP_CHECK(hipGetLastError());
     return SHP_OK;
 }

@@ -365,7 +365,8 @@ int shp_workspace_info(shp_ctx* ctx, void** dptr, uint64_t* bytes) {
 // ir_cout_splits and the model graphs' ir_fuse; conv_direct (-1: small-channel 3x3
 // conv2d_nhwc on the implicit GEMM instead of the direct kernel); gemm_small (1x1 conv2d_nhwc
 // on the small-product kernel: 1 wherever it fits, k >= 2 with k K-splits, -1 never); fc_mfma (-1:
-// fully_connected with 2-16 rows on the wavefront-per-column or tiled kernels).
+// fully_connected with 2-16 rows on the wavefront-per-column or tiled kernels); direct (products
+// and convolutions on the small-problem kernel with k K-splits, -1 never).
 int shp_tune(shp_ctx* ctx, const char* key, int value) {
     if (!ctx) return fail(SHP_ERR_INVALID, "shp_tune: null ctx");
     shp::GemmTune& t = reinterpret_cast<Ctx*>(ctx)->tune;
@@ -389,6 +390,7 @@ int shp_tune(shp_ctx* ctx, const char* key, int value) {
     else if (k == "conv_direct") t.conv_direct = value;
     else if (k == "gemm_small") t.small = value;
     else if (k == "fc_mfma") t.fc = value;
+    else if (k == "direct") t.direct = value;
     else return fail(SHP_ERR_INVALID, "shp_tune: unknown key '" + k + "'");
     return SHP_OK;
 }

@@ -985,6 +985,57 @@ def test_hlo_shape_ops_fail_closed(ctx):
         _dev(ctx, "hlo_slice", rnd(4, 6), None, 5, H.slice_push((4, 6), (0, 0), (2, 6)))
 
 
+DIRECT_DOTS = [(1, 16, 4), (5, 48, 68), (32, 128, 64), (33, 144, 132), (64, 2048, 200), (97, 400, 1000),
+               (250, 768, 320)]
+
+
+@pytest.mark.parametrize("splits", [1, 2, 3, 8])
+@pytest.mark.parametrize("m,k,n", DIRECT_DOTS)
+def test_gemm_direct_products(ctx, orc, m, k, n, splits):
+    """The small-problem kernel on [K][N] and [N][K] operands: row and column tails, fewer K steps
+    than wavefronts, K splits (bit-identical repeats), bias, residual and activation."""
+    x, w, b, r = rnd(m, k), rnd(k, n), rnd(n), rnd(m, n)
+    push = [m, k, n, m * n]
+    ctx.tune("direct", splits)
+    try:
+        y, ref = both(ctx, orc, "hlo_dot_rank2", x, w, m * n, push, bias=b, residual=r, act="relu")
+        assert_close(y, ref, 1e-4, 1e-4, "direct [K][N]")
+        y2, _ = both(ctx, orc, "hlo_dot_rank2", x, w, m * n, push, bias=b, residual=r, act="relu")
+        np.testing.assert_array_equal(y, y2)
+        strides = [1, 1, m, n, k, 0, 0, k, 1, 0, 0, 1, k, 0, 0, n, 1]
+        y, ref = both(ctx, orc, "dot_general_strided", x, np.ascontiguousarray(w.T), m * n, strides,
+                      bias=b, residual=r, act="silu")
+        assert_close(y, ref, 1e-4, 1e-4, "direct [N][K]")
+    finally:
+        ctx.tune("direct", 0)
+
+
+@pytest.mark.parametrize("n,ih,ic,k,oc,s", [(1, 7, 16, 3, 36, 1), (3, 9, 48, 3, 64, 2), (2, 14, 32, 1, 100, 1),
+                                            (1, 13, 64, 5, 64, 2), (5, 14, 256, 3, 256, 1), (2, 8, 64, 1, 64, 2)])
+def test_gemm_direct_convolutions(ctx, orc, n, ih, ic, k, oc, s):
+    """The same on NHWC convolutions: padding taps, tap changes inside a wavefront's K range, strides;
+    HWIO weights forced at 1 and 4 splits, and by the planner's own choice."""
+    p = (k - 1) // 2
+    oh = (ih + 2 * p - k) // s + 1
+    x, w = rnd(n, ih, ih, ic), rnd(k, k, ic, oc) * np.float32(np.sqrt(2.0 / (k * k * ic)))
+    b, r = rnd(oc), rnd(n, oh, oh, oc)
+    total = n * oh * oh * oc
+    push = [n, ih, ih, ic, k, k, oc, oh, oh, s, s, p, p, total]
+    wt = np.ascontiguousarray(w.transpose(3, 0, 1, 2))
+    push2 = [n, ic, ih, ih, oc, oh, oh, k, k, s, s, 1, p, p, total]
+    for splits in (1, 4, 0):
+        ctx.tune("direct", splits)
+        ctx.tune("gemm_small", -1)
+        try:
+            y, ref = both(ctx, orc, "hlo_conv_nhwc_hwio", x, w, total, push, bias=b, residual=r, act="relu")
+            assert_close(y, ref, 1e-4, 1e-4, f"direct HWIO, {splits} splits")
+            y, ref = both(ctx, orc, "conv2d_nhwc", x, orc.pack_conv_weight(wt, b), total, push2, act="relu6")
+            assert_close(y, ref, 1e-4, 1e-4, f"direct OHWI, {splits} splits")
+        finally:
+            ctx.tune("direct", 0)
+            ctx.tune("gemm_small", 0)
+
+
 @pytest.mark.parametrize("n", [1, 3, 1000, 131073, 262143, 262144, 262145, 300001, (16 << 20) + 5])
 def test_run_kernel_sizes(n):
     """Host buffers in and out around the pinned-staging (1 MiB each way) and kept-buffer (64 MiB)
