@@ -714,7 +714,7 @@ static const char* kNames[] = {
     "hlo_dot_rank2", "conv2d_nhwc", "dot_general_strided", "depthwise_conv2d",
     "resize_bilinear", "depthwise_conv2d_nhwc", "gemv_nt", "argmax_rows", "gather_rows", "hlo_broadcast",
     "hlo_transpose", "hlo_slice", "hlo_concatenate_into", "hlo_compare", "hlo_select",
-    "hlo_reduce", "hlo_strided_copy", "attention_fused", "nan_count", "inverted_residual_nhwc",
+    "hlo_reduce", "hlo_strided_copy", "attention_fused", "attention_rows", "nan_count", "inverted_residual_nhwc",
     "conv1x1_gap_nhwc"};
 
 int orc_kernel_count(void) { return (int)(sizeof kNames / sizeof kNames[0]); }
@@ -1002,7 +1002,7 @@ int orc_run_kernel(const char* name, const float* in0, size_t n0, const float* i
                     q[11], q[12], out, q[13], q[14], q[15], q[16], bias, residual, act, alpha);
         return 0;
     }
-    if (!strcmp(name, "attention_fused")) {
+    if (!strcmp(name, "attention_fused") || !strcmp(name, "attention_rows")) {
         /* {B, H, S, HD, ld_in, q_off, k_off, v_off, ld_out, scale_bits, total = B*S*ld_out} */
         NEED(11);
         const int32_t* q = push;

@@ -1,4 +1,5 @@
-// Blocked attention over any sequence length (head dim 64), used by the decoder's prompt pass.
+// Attention over any sequence length (head dim 64): attention_rows, attention_fused and the
+// decoder's prompt pass.
 #pragma once
 
 #include "common.h"
@@ -10,7 +11,7 @@ namespace shp {
 // Rows are 64 contiguous floats, 16-byte aligned.
 struct AttnArgs {
     const float *q, *k, *v;
-    const float* mask;  // [n_keys] additive, or null
+    const float* mask;  // [n_keys] additive, or null (not with causal)
     float* out;
     int64_t q_b, q_h, q_r, k_b, k_h, k_r, v_b, v_h, v_r, o_b, o_h, o_r;
     int batch, kv_heads, group;  // group query heads share one KV head

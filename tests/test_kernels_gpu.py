@@ -633,6 +633,30 @@ def test_attention_fused(ctx, orc, B, H, masked, pad_out):
     assert_close(y[cols], r[cols], 1e-4, 1e-4, f"attention_fused {push[:9]}")
 
 
+@pytest.mark.parametrize("S", [1, 5, 16, 17, 63, 64, 65, 127, 129, 200, 321])
+@pytest.mark.parametrize("masked", ["none", "random", "lowest"])
+def test_attention_rows(ctx, orc, S, masked):
+    """Any sequence: query and key tails of the 16-query and 64/128-key blocks, an additive mask with
+    keys hidden by the lowest float (all of them in the second batch's case), unaligned output rows."""
+    B, H, HD, pad = 2, 3, 64, 1 if S % 2 else 0
+    D = H * HD
+    qkv = rnd(B * S, 3 * D)
+    mask = None
+    if masked == "random":
+        mask = rnd(S, scale=0.5)
+    elif masked == "lowest":
+        mask = np.zeros(S, np.float32)
+        mask[S // 2:] = np.finfo(np.float32).min
+        if S == 5:
+            mask[:] = np.finfo(np.float32).min  # every key hidden: the row is uniform
+    ld_out = D + pad
+    sb = int(np.array([0.125], np.float32).view(np.int32)[0])
+    push = [B, H, S, HD, 3 * D, 0, D, 2 * D, ld_out, sb, B * S * ld_out]
+    y, r = both(ctx, orc, "attention_rows", qkv, mask, B * S * ld_out, push)
+    cols = np.arange(B * S * ld_out) % ld_out < D
+    assert_close(y[cols], r[cols], 1e-4, 1e-4, f"attention_rows S={S} {masked}")
+
+
 def test_attention_fused_rejects_other_sequence_lengths(ctx):
     from spirv_inference_amd import ShpError
     S, HD, B, H = 64, 64, 1, 2

@@ -144,6 +144,21 @@ def test_bert_base_per_op(ctx, orc):
                      "bert final hidden (chained)")
 
 
+@pytest.mark.parametrize("batch,seq", [(3, 200), (1, 17)])
+def test_bert_base_other_sequences(ctx, orc, batch, seq):
+    """Sequences that are not 128 (attention_rows instead of attention_fused), per op and chained."""
+    from oracle import walk
+    from spirv_inference_amd.models import Model
+    with Model(ctx, "bert_base", batch, seq_len=seq, seed=2) as m:
+        m.run()
+        ctx.sync()
+        assert sum(o.kernel == "attention_rows" for o in m.ops()) == 12
+        check_per_op(m, walk)
+        host = walk.chained(m)
+        assert_close(m.output(0).download(), host[m.ops()[-1].out], 1e-3, 1e-3,
+                     "bert final hidden (chained)")
+
+
 def test_resnet50_b32_graph_replay_and_top1(ctx, orc):
     """The benchmark config: graph replays equal the eager result; top-1 equals the oracle's."""
     from oracle import walk
