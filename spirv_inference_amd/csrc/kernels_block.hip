@@ -686,8 +686,8 @@ double plan_cost(const IrShape& sh, const IrGeom& g) {
 // split and output-channel slice per block, each timed as 20 launches of the block replayed
 // from a hipGraph, beside the three operators conv2d_nhwc, depthwise_conv2d_nhwc, conv2d_nhwc
 // timed the same way), and whether one launch beat the three operators; where the two were
-// close the whole model's graph replay decided.  The cost model and the rule of fusion_pays
-// cover every other shape.
+// close the whole model's graph replay decided.  The cost model (at batches 2-32 its plans lie
+// within 4 % of a sweep's best) and the rules of fusion_pays cover every other shape.
 struct TunedBlock {
     int n, cin, h, w, ce, cout, k, s, expand;
     int th, tw, S, J;
@@ -739,13 +739,33 @@ const TunedBlock* tuned_block(const IrShape& sh) {
     return nullptr;
 }
 
-// Whether one launch is expected to beat the three-operator form: the measured verdict for
-// the blocks above; elsewhere, for blocks with an expand, where the separate launches are
-// latency-bound (at most 1024 output pixels in the batch) or the expand is a thin,
-// memory-bound product (cin <= 48) whose output the fused form never writes.
+// Whether one launch is expected to beat the separate ones: the measured verdict for the blocks
+// above; elsewhere rules on sizes, fitted to the 21 distinct blocks of MobileNetV2 and
+// EfficientNet-Lite0 at batches 1-32, each as one launch, as expand GEMM + depthwise/projection
+// launch and as three launches (graph-replayed; the rules' sums lie within 4 % of the fastest form
+// per block at every batch).  A whole block pays
+// * with cin <= 24 at any size: the expand is thin and memory bound, its output six times the input;
+// * with cin <= 48 up to 2,000 input pixels (1x28x28x32: 10.0 us against 12.8 in three launches;
+//   4x28x28x32 to 64: 17.5 against 13.7);
+// * beyond, where the launches are latencies: 3x3, ce under 900, cin * pixels up to 37,000
+//   (1x14x14x96: 14.0 against 14.7; 4x14x14x96: 22.1 against 18.8; 12x7x7x192: 63.2 against 27.9).
+// The depthwise + projection form (no expand) pays with ce <= 96 at any size; at stride 1 up to ce
+// 256 (24x56x56x144: 0.87 of the two launches) and up to ce 700 while the projection is small
+// (4x14x14x384: 0.95, 12x14x14x384: 1.15); at stride 2 up to ce 256 for few outputs, more of them
+// with a 5x5 window, whose taps the fused form reads from LDS.
 bool fusion_pays(const IrShape& sh) {
     if (const TunedBlock* t = tuned_block(sh)) return t->fuse;
-    return sh.expand && ((int64_t)sh.n * sh.oh * sh.ow <= 1024 || sh.cin <= 48);
+    const int64_t in = (int64_t)sh.n * sh.h * sh.w, out = (int64_t)sh.n * sh.oh * sh.ow;
+    if (sh.expand) {
+        if (sh.cin <= 24) return true;
+        if (sh.cin <= 48) return in <= 2000;
+        return sh.k == 3 && sh.ce < 900 && sh.cin * in <= 37000;
+    }
+    if (sh.ce <= 96) return true;
+    if (sh.s == 1)
+        return sh.ce <= 256 || (sh.ce <= 480 && out <= (sh.k == 5 ? 1600 : 1200)) ||
+               (sh.ce <= 700 && out <= 800);
+    return sh.ce <= 256 && out <= (sh.k == 5 ? 6300 : 400);
 }
 
 IrPlan choose_plan(const IrShape& sh, const shp::GemmTune& tn, bool allow_split) {
