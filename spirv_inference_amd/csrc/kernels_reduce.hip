@@ -511,41 +511,79 @@ __global__ __launch_bounds__(256) void softmax_rows_kernel(const float* __restri
     }
 }
 
-// One wavefront per row for short rows (attention scores of length <= 1024).
+// One wavefront per row for rows of up to 2,048 (1,024 without 16-byte loads: 32 single floats a
+// lane took 24 us on 7,000x1,501, a workgroup per row 21): the row is read once and stays in registers, N
+// elements of W (16-byte loads, or single floats where the length or alignment does not allow them)
+// per lane, all loads in flight at once; the maximum and the sum are lane exchanges, no LDS and no
+// barrier.  Element c of slot j of a lane is column (j * 64 + lane) * W + c.
+typedef float rowvec4 __attribute__((ext_vector_type(4)));
+template <int W>
+__device__ __forceinline__ void row_load(const float* p, int i, int cols, float (&v)[W], float fill) {
+    if constexpr (W == 4) {
+        const rowvec4 t = i < cols ? *reinterpret_cast<const rowvec4*>(p + i) : rowvec4{fill, fill, fill, fill};
+        v[0] = t.x; v[1] = t.y; v[2] = t.z; v[3] = t.w;
+    } else {
+        v[0] = i < cols ? p[i] : fill;
+    }
+}
+template <int W>
+__device__ __forceinline__ void row_store(float* p, int i, int cols, const float (&v)[W]) {
+    if (i >= cols) return;
+    if constexpr (W == 4) *reinterpret_cast<rowvec4*>(p + i) = rowvec4{v[0], v[1], v[2], v[3]};
+    else p[i] = v[0];
+}
+
+template <int W, int N>
 __global__ __launch_bounds__(256) void softmax_rows_wave_kernel(const float* __restrict__ x,
                                                                 const float* __restrict__ mask,
                                                                 float* __restrict__ y, int rows,
                                                                 int cols, float scale) {
-    int lane = threadIdx.x & 63;
-    int wave = blockIdx.x * 4 + (threadIdx.x >> 6);
-    int nwaves = gridDim.x * 4;
-    constexpr int kMaxPer = 16;
-    for (int r = wave; r < rows; r += nwaves) {
+    const int lane = threadIdx.x & 63;
+    const int nwaves = gridDim.x * 4;
+    for (int r = blockIdx.x * 4 + (threadIdx.x >> 6); r < rows; r += nwaves) {
         const float* xr = x + (uint64_t)r * cols;
         float* yr = y + (uint64_t)r * cols;
-        float v[kMaxPer];
+        float v[N][W];
+#pragma unroll
+        for (int j = 0; j < N; ++j) row_load<W>(xr, (j * 64 + lane) * W, cols, v[j], 0.0f);
         float m = kNegMax;
 #pragma unroll
-        for (int j = 0; j < kMaxPer; ++j) {
-            int i = lane + j * 64;
-            v[j] = i < cols ? xr[i] * scale + (mask ? mask[i] : 0.0f) : kNegMax;
-            m = fmaxf(m, v[j]);
+        for (int j = 0; j < N; ++j) {
+            const int i = (j * 64 + lane) * W;
+            float t[W];
+#pragma unroll
+            for (int c = 0; c < W; ++c) t[c] = 0.0f;
+            if (mask) row_load<W>(mask, i, cols, t, 0.0f);
+#pragma unroll
+            for (int c = 0; c < W; ++c) {
+                v[j][c] = i < cols ? v[j][c] * scale + t[c] : kNegMax;
+                m = fmaxf(m, v[j][c]);
+            }
         }
         m = wave_max(m);
         float s = 0.0f;
 #pragma unroll
-        for (int j = 0; j < kMaxPer; ++j) {
-            int i = lane + j * 64;
-            v[j] = i < cols ? expf(v[j] - m) : 0.0f;
-            s += v[j];
+        for (int j = 0; j < N; ++j) {
+            const int i = (j * 64 + lane) * W;
+#pragma unroll
+            for (int c = 0; c < W; ++c) {
+                v[j][c] = i < cols ? expf(v[j][c] - m) : 0.0f;
+                s += v[j][c];
+            }
         }
         s = wave_sum(s);
 #pragma unroll
-        for (int j = 0; j < kMaxPer; ++j) {
-            int i = lane + j * 64;
-            if (i < cols) yr[i] = v[j] / s;
+        for (int j = 0; j < N; ++j) {
+#pragma unroll
+            for (int c = 0; c < W; ++c) v[j][c] = v[j][c] / s;
+            row_store<W>(yr, (j * 64 + lane) * W, cols, v[j]);
         }
     }
+}
+
+// The row kernels' mask or weight rows must be aligned as the data for 16-byte loads.
+inline bool rows_vec(const shp::Launch& l, int cols) {
+    return cols % 4 == 0 && (((uintptr_t)l.in0 | (uintptr_t)l.in1 | (uintptr_t)l.out) & 15) == 0;
 }
 
 int launch_softmax_rows(const shp::Launch& l) {
@@ -557,10 +595,19 @@ int launch_softmax_rows(const shp::Launch& l) {
     float scale;
     int32_t bits = l.push[2];
     memcpy(&scale, &bits, 4);
-    if (cols <= 1024) {
-        hipLaunchKernelGGL(softmax_rows_wave_kernel, dim3(cap_grid(rows, 4)), dim3(256), 0,
-                           l.stream, (const float*)l.in0, (const float*)l.in1, (float*)l.out,
-                           rows, cols, scale);
+    const bool vec = rows_vec(l, cols);
+    if (cols <= (vec ? 2048 : 1024)) {
+        auto kern = vec
+                        ? (cols <= 256    ? softmax_rows_wave_kernel<4, 1>
+                           : cols <= 512  ? softmax_rows_wave_kernel<4, 2>
+                           : cols <= 1024 ? softmax_rows_wave_kernel<4, 4>
+                                          : softmax_rows_wave_kernel<4, 8>)
+                        : (cols <= 256    ? softmax_rows_wave_kernel<1, 4>
+                           : cols <= 512  ? softmax_rows_wave_kernel<1, 8>
+                                          : softmax_rows_wave_kernel<1, 16>);
+        hipLaunchKernelGGL(kern, dim3(cap_grid(rows, 4)), dim3(256), 0, l.stream,
+                           (const float*)l.in0, (const float*)l.in1, (float*)l.out, rows, cols,
+                           scale);
     } else {
         unsigned g = rows < 65536 ? rows : 65536;
         hipLaunchKernelGGL(softmax_rows_kernel, dim3(g), dim3(256), 0, l.stream,
@@ -575,7 +622,7 @@ int launch_softmax_rows(const shp::Launch& l) {
 // layernorm: y = (x - mean) * rsqrt(var + eps) * gamma + beta, var = mean((x-mean)^2);
 //            in1 = [gamma(cols) | beta(cols)]  (BERT, eps 1e-12)
 // rmsnorm:   y = x * rsqrt(mean(x^2) + eps) * w; in1 = w(cols)   (export_llama.py:284-286)
-// push {rows, cols, eps_bits}.  One 256-thread group per row, fp32 accumulation.
+// push {rows, cols, eps_bits}.  Rows past 2,048: one 256-thread group each, fp32 accumulation.
 template <bool RMS>
 __global__ __launch_bounds__(256) void rownorm_kernel(const float* __restrict__ x,
                                                       const float* __restrict__ w,
@@ -605,6 +652,57 @@ __global__ __launch_bounds__(256) void rownorm_kernel(const float* __restrict__ 
     }
 }
 
+// The same with one wavefront per row of up to 2,048, the row in registers (see
+// softmax_rows_wave_kernel): one pass over memory where a workgroup per row made three (16,000x2,048:
+// 80 -> 44 us).
+template <bool RMS, int W, int N>
+__global__ __launch_bounds__(256) void rownorm_wave_kernel(const float* __restrict__ x,
+                                                           const float* __restrict__ w,
+                                                           float* __restrict__ y, int rows, int cols,
+                                                           float eps) {
+    const int lane = threadIdx.x & 63;
+    const int nwaves = gridDim.x * 4;
+    for (int r = blockIdx.x * 4 + (threadIdx.x >> 6); r < rows; r += nwaves) {
+        const float* xr = x + (uint64_t)r * cols;
+        float* yr = y + (uint64_t)r * cols;
+        float v[N][W];
+#pragma unroll
+        for (int j = 0; j < N; ++j) row_load<W>(xr, (j * 64 + lane) * W, cols, v[j], 0.0f);
+        float mean = 0.0f;
+        if constexpr (!RMS) {
+            float s = 0.0f;
+#pragma unroll
+            for (int j = 0; j < N; ++j)
+#pragma unroll
+                for (int c = 0; c < W; ++c) s += v[j][c];
+            mean = wave_sum(s) / (float)cols;
+        }
+        float ss = 0.0f;
+#pragma unroll
+        for (int j = 0; j < N; ++j)
+#pragma unroll
+            for (int c = 0; c < W; ++c) {
+                const float d = (j * 64 + lane) * W < cols ? v[j][c] - mean : 0.0f;
+                ss += d * d;
+            }
+        const float inv = 1.0f / sqrtf(wave_sum(ss) / (float)cols + eps);
+#pragma unroll
+        for (int j = 0; j < N; ++j) {
+            const int i = (j * 64 + lane) * W;
+            float g[W], b[W];
+            row_load<W>(w, i, cols, g, 0.0f);
+            if constexpr (!RMS) row_load<W>(w + cols, i, cols, b, 0.0f);
+#pragma unroll
+            for (int c = 0; c < W; ++c) {
+                const float t = (v[j][c] - mean) * inv;
+                if constexpr (RMS) v[j][c] = t * g[c];
+                else v[j][c] = t * g[c] + b[c];
+            }
+            row_store<W>(yr, i, cols, v[j]);
+        }
+    }
+}
+
 template <bool RMS>
 int launch_rownorm(const shp::Launch& l) {
     if (l.n_push < 3) return shp::fail(SHP_ERR_PUSH, "row norm needs {rows, cols, eps_bits}");
@@ -616,6 +714,21 @@ int launch_rownorm(const shp::Launch& l) {
     float eps;
     int32_t bits = l.push[2];
     memcpy(&eps, &bits, 4);
+    const bool vec = rows_vec(l, cols);
+    if (cols <= (vec ? 2048 : 1024)) {
+        auto kern = vec
+                        ? (cols <= 256    ? rownorm_wave_kernel<RMS, 4, 1>
+                           : cols <= 512  ? rownorm_wave_kernel<RMS, 4, 2>
+                           : cols <= 1024 ? rownorm_wave_kernel<RMS, 4, 4>
+                                          : rownorm_wave_kernel<RMS, 4, 8>)
+                        : (cols <= 256    ? rownorm_wave_kernel<RMS, 1, 4>
+                           : cols <= 512  ? rownorm_wave_kernel<RMS, 1, 8>
+                                          : rownorm_wave_kernel<RMS, 1, 16>);
+        hipLaunchKernelGGL(kern, dim3(cap_grid(rows, 4)), dim3(256), 0, l.stream,
+                           (const float*)l.in0, (const float*)l.in1, (float*)l.out, rows, cols, eps);
+        SHP_HIP_CHECK(hipGetLastError());
+        return SHP_OK;
+    }
     unsigned g = rows < 65536 ? rows : 65536;
     hipLaunchKernelGGL((rownorm_kernel<RMS>), dim3(g), dim3(256), 0, l.stream,
                        (const float*)l.in0, (const float*)l.in1, (float*)l.out, rows, cols, eps);

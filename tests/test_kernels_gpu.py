@@ -1001,6 +1001,75 @@ def test_hlo_reduce(ctx, orc, shape, dims):
                                       orc.run("hlo_reduce", x, None, kept, push))
 
 
+@pytest.mark.parametrize("cols", [1, 3, 4, 63, 64, 100, 255, 256, 260, 511, 768, 1001, 1024, 1028, 2047, 2048, 2052, 3001])
+@pytest.mark.parametrize("rows", [1, 5, 130])
+def test_row_kernels_all_widths(ctx, orc, rows, cols):
+    """Every register-resident width of the row kernels (16-byte and single-float loads), the wide
+    fallback, masked softmax with hidden columns, a mask offset by one float (unaligned)."""
+    x, w = rnd(rows, cols) * 2, rnd(2 * cols)
+    sb = int(np.array([0.5], np.float32).view(np.int32)[0])
+    eb = int(np.array([1e-12], np.float32).view(np.int32)[0])
+    mask = rnd(cols)
+    mask[cols // 2 + 1:] = np.finfo(np.float32).min
+    for k, b, push in (("layernorm_rows", w, [rows, cols, eb]), ("rmsnorm_rows", w[:cols], [rows, cols, eb]),
+                       ("softmax_rows", None, [rows, cols, sb]), ("softmax_rows", mask, [rows, cols, sb])):
+        if cols == 1 and k == "layernorm_rows":
+            continue  # zero variance: rounding over sqrt(1e-12)
+        y, r = both(ctx, orc, k, x, b, rows * cols, push)
+        assert_close(y, r, 1e-4, 1e-4, f"{k} {rows}x{cols}")
+
+
+GATHERS = [((3, 5, 7, 64), (0, 2, 1, 3)), ((3, 5, 7, 33), (0, 2, 1, 3)), ((2, 70, 12, 64), (0, 2, 3, 1)),
+           ((2, 70, 12, 33), (0, 3, 2, 1)), ((1, 300, 4, 64), (0, 1, 3, 2)), ((7, 9, 130, 3), (2, 0, 1, 3)),
+           ((65, 129), (1, 0)), ((300, 5), (1, 0)), ((5, 300), (1, 0)), ((2, 3, 2, 5, 3, 4), (5, 0, 3, 1, 4, 2)),
+           ((64, 64, 1, 16), (3, 2, 1, 0)), ((8,), (0,)), ((1, 1), (1, 0)), ((4, 257, 66), (2, 1, 0))]
+
+
+@pytest.mark.parametrize("shape,perm", GATHERS)
+def test_gather_forms_transpose(ctx, orc, shape, perm):
+    """Row, tile and generic forms of the strided gather: merged axes, tails, axes shorter and longer
+    than a tile, also from a source that is only 4-byte aligned."""
+    from spirv_inference_amd import hlo_ops as H
+    n = int(np.prod(shape))
+    x, push = rnd(*shape), H.transpose_push(shape, perm)
+    want = orc.run("hlo_transpose", x, None, n, push)
+    np.testing.assert_array_equal(_dev(ctx, "hlo_transpose", x, None, n, push), want)
+    from spirv_inference_amd.runtime import DeviceTensor
+    big, out = ctx.tensor(np.concatenate([[0], x.ravel()])), ctx.empty(n + 1)
+    ctx.launch("hlo_transpose", DeviceTensor(ctx, n, ptr=big.ptr + 4, owned=False), None,
+               DeviceTensor(ctx, n, ptr=out.ptr + 4, owned=False), push)
+    ctx.sync()
+    np.testing.assert_array_equal(out.download()[1:], want)
+    for t in (big, out):
+        t.free()
+
+
+@pytest.mark.parametrize("op", range(8))
+@pytest.mark.parametrize("dims,sa,sb", [((1, 1, 50, 64), (0, 0, 64, 1), (0, 0, 0, 1)),
+                                        ((2, 3, 5, 8), (120, 40, 8, 1), (0, 1, 0, 0)),
+                                        ((2, 3, 5, 8), (0, 0, 0, 1), (120, 40, 8, 1)),
+                                        ((1, 7, 1, 12), (0, 12, 0, 1), (0, 1, 0, 0)),
+                                        ((3, 4, 5, 6), (120, 30, 6, 1), (0, 0, 6, 1)),
+                                        ((2, 2, 3, 4), (3, 0, 1, 0), (0, 12, 4, 1)),
+                                        ((1, 1, 9, 20), (0, 0, 21, 1), (0, 0, 0, 0))])
+def test_broadcast_binary_forms(ctx, orc, op, dims, sa, sb):
+    n = int(np.prod(dims))
+    size = lambda st: 1 + sum((d - 1) * s for d, s in zip(dims, st))
+    a, b = np.abs(rnd(size(sa))) + 0.5, np.abs(rnd(size(sb))) + 0.5
+    push = [op, n, *dims, *sa, *sb]
+    y, r = both(ctx, orc, "broadcast_binary", a, b, n, push)
+    assert_close(y, r, 1e-5, 1e-5, f"broadcast_binary {push}")
+
+
+@pytest.mark.parametrize("n,c", [(12, 4), (3000, 12), (4096, 1024), (70, 7), (8 * 1028, 1028)])
+@pytest.mark.parametrize("act", ["none", "relu6", "gelu_erf"])
+def test_bias_act_forms(ctx, orc, n, c, act):
+    x, b, res = rnd(n), rnd(c), rnd(n)
+    for kw in (dict(bias=b), dict(bias=b, residual=res), dict(residual=res)):
+        y, r = both(ctx, orc, "bias_act", x, None, n, [n, c], act=act, **kw)
+        assert_close(y, r, 1e-5, 1e-5, f"bias_act {n} {c} {act}")
+
+
 def test_hlo_shape_ops_fail_closed(ctx):
     from spirv_inference_amd import hlo_ops as H
     with pytest.raises(RuntimeError):  # not a permutation
