@@ -552,7 +552,8 @@ int shp_llama_generate(shp_llama* p, const int32_t* prompt, int32_t n_prompt, in
     if (n_prompt + n_new - 1 > lm->cfg.max_seq)
         return fail(SHP_ERR_SHAPE, "shp_llama_generate: prompt + new tokens exceed max_seq");
     int rc = lm->reset();
-    if (n_prompt > 1 && lm->pf_rows) {
+    // a pass over 2-16 rows takes 1.65-1.9 ms, a token step 0.77: the pass from three ids on
+    if (n_prompt > 2 && lm->pf_rows) {
         for (int i = 0; i < n_prompt && !rc; ++i)
             if (prompt[i] < 0 || prompt[i] >= lm->cfg.vocab)
                 rc = fail(SHP_ERR_SHAPE, "shp_llama_step: token id");
