@@ -2142,6 +2142,7 @@ int launch_stem(hipStream_t s, const GemmParams& p) {
 struct Plan {
     TileCfg t;
     int splits, kps;
+    double cost;  // seconds by bl_plan_cost, 0 for plans of the other kernels and of the table
 };
 
 // Workgroups resident per CU, as the compiler reports them for each variant (LDS of the
@@ -2163,7 +2164,6 @@ int occupancy(TileCfg t) {
 // and the twice higher residency of the 16-deep tile wins (K = 64..256 layers measured
 // 3-16 % faster with it).
 double tile_eff(TileCfg t, int kps) {
-    if (t.bl) return t.bk == 16 && kps > 256 ? 0.85 : 1.0;
     if (t.dma) return 1.1;
     double e = (t.bm == 128 && t.bn == 128) ? 1.0 : 0.85;
     return t.bk == 16 && kps > 256 ? e * 0.85 : e;
@@ -2174,19 +2174,57 @@ double tile_eff(TileCfg t, int kps) {
 // reduction pass.
 double plan_cost(const GemmParams& p, int nbatch, TileCfg t, int splits, int kps) {
     static const double kUtil[8] = {0.4, 0.6, 0.75, 0.85, 0.9, 0.92, 0.95, 1.0};
-    // the buffer-loaded kernel keeps its own MFMA stream fed: one workgroup per CU already
-    // runs at ~80 % of the CU's rate (MI355X, 1568x512x4608 on 200 CUs)
-    static const double kUtilBl[8] = {0.8, 0.9, 0.94, 0.96, 0.97, 0.98, 0.99, 1.0};
     const double cu_rate = 256.0 * 2.4e9;  // fp32 MFMA FLOP/s per CU
     int64_t tiles = (int64_t)((p.M + t.bm - 1) / t.bm) * ((p.N + t.bn - 1) / t.bn) * nbatch;
     int64_t wgs = tiles * splits;
     int64_t per_cu = (wgs + 255) / 256;
     int resident = (int)std::min<int64_t>(occupancy(t), per_cu);
-    double util = (t.bl ? kUtilBl : kUtil)[std::min(resident, 8) - 1];
+    double util = kUtil[std::min(resident, 8) - 1];
     double wg_flops = 2.0 * t.bm * t.bn * kps;
     double cost = per_cu * wg_flops / (cu_rate * tile_eff(t, kps) * util);
     if (splits > 1) cost += (splits + 1.0) * p.M * (double)p.N * nbatch * 4.0 / 3.0e12 + 2.0e-6;
     return cost;
+}
+
+// Estimated time of a plan of the buffer-loaded kernel, and of the direct kernel's unsplit plan in
+// the same unit.  Fitted over 526 products and convolutions with more than 256 32x64 tiles
+// (130-16,384 rows of 64-4,096 k; 1x1, 3x3 and 5x5 over 56^2-7^2 maps of 32-2,048 channels at
+// batches 1-32; multiples of the tiles and not), every tile, K tile and split count of each
+// measured: the chosen plan is 0.9 % slower than the best one on average.  The rule before it (no
+// fixed costs, the 16-deep K tile charged 15 % of its rate on long loops, never the direct kernel)
+// was 4.6 % slower over the half of them it was timed on and lost up to 1.3 times: 1200x1000x2048
+// 61.8 -> 51.9 us (a 16-deep tile in 4 splits), 3x3 over 20x14x14x256 58.0 -> 44.7 (direct).
+//  - One workgroup per CU runs at 0.76 of the MFMA rate, two at 0.815, as many as fit at 1,
+//    and 32-deep 64x64 tiles, four of which fit, at 1 from eight to a CU on (4096x3072x768: 147 us,
+//    160 with the 16-deep tile).  Gathers with taps run at 1 / 1.58 of a product's rate.
+//  - The 16-deep K tile's higher residency wins 8 % on at most 256 k; beyond, K tiles tie, but
+//    with the short chains' second sums it runs at 0.85 (512-row prompt pass 10.5 ms, 11.4 without).
+//  - A split writes and reads its partial sums and pays the counters' round trip.
+//  - The direct kernel's 32x64 tiles fill the rounds that 64x64 tiles leave half empty (600 tiles
+//    are 3 rounds of half the work, 300 are 2), but each round pays its pipeline's fill, which is
+//    what a short K does not earn back.  250 tiles a round: a round within a few tiles of full
+//    takes as long as one more.
+constexpr double kCuRate = 256.0 * 2.4e9;  // fp32 MFMA FLOP/s per CU
+
+double bl_plan_cost(const GemmParams& p, int nbatch, int amode, TileCfg t, int splits, int kps) {
+    static const double kUtil[5] = {0.76, 0.815, 0.93, 0.95, 1.0};
+    int64_t tiles = (int64_t)((p.M + t.bm - 1) / t.bm) * ((p.N + t.bn - 1) / t.bn) * nbatch;
+    int64_t per_cu = (tiles * splits + 255) / 256;
+    int resident = (int)std::min<int64_t>(occupancy(t), per_cu);
+    if (t.bk == 32 && t.bm == 64 && per_cu >= 8) resident = 5;
+    double rate = kCuRate * kUtil[std::min(resident, 5) - 1];
+    if (t.bk == 16) rate *= kps <= 256 ? 1.08 : p.short_chains ? 0.85 : 1.0;
+    if (amode == shp::A_CONV_NHWC4 && p.ckh * p.ckw > 1) rate /= 1.58;
+    double cost = 1.0e-6 + per_cu * (0.3e-6 + 2.0 * t.bm * t.bn * kps / rate);
+    if (splits > 1) cost += 1.45 * splits * p.M * (double)p.N * nbatch * 4.0 / 3.0e12 + 4.1e-6;
+    return cost;
+}
+
+double direct_cost(const GemmParams& p, int amode) {
+    const bool conv = amode == shp::A_CONV_NHWC4;
+    int64_t tiles = (int64_t)((p.M + 31) / 32) * ((p.N + 63) / 64);
+    double round = (conv ? 3.5e-6 : 0.8e-6) + 2.0 * 32 * 64 * p.K / kCuRate * (conv ? 1.18 : 1.41);
+    return 1.0e-6 + (double)((tiles + 249) / 250) * round;
 }
 
 // Plans measured best on MI355X for the benchmark configs' shapes: sweeps of every tile, K
@@ -2253,7 +2291,7 @@ bool tuned_plan(const GemmParams& p, int nbatch, int amode, int bmode, bool hot,
         const int kq = t.bl && t.bk == 64 ? 64 : 32;
         int kps = ((p.K + e.splits - 1) / e.splits + kq - 1) / kq * kq;
         if ((p.K + kps - 1) / kps != e.splits) return false;
-        *out = Plan{t, e.splits, kps};
+        *out = Plan{t, e.splits, kps, 0};
         return true;
     }
     return false;
@@ -2263,11 +2301,12 @@ const int kSplits[] = {1, 2, 3, 4, 5, 6, 8, 12, 16};
 
 // The buffer-loaded kernel's plan: tile, K tile and split count by the cost model, among the
 // K tiles of `blm` (bl_mask) and the tune overrides.  False when no candidate fits.
-bool plan_bl(const GemmParams& p, int nbatch, int blm, const shp::GemmTune& tn, Plan* out) {
+bool plan_bl(const GemmParams& p, int nbatch, int amode, int blm, const shp::GemmTune& tn,
+             Plan* out) {
     static const TileCfg kBl[] = {{128, 128, 32, false, 1, true}, {128, 64, 32, false, 1, true},
                                   {64, 64, 64, false, 1, true},   {64, 64, 32, false, 1, true},
                                   {64, 64, 16, false, 1, true}};
-    Plan best{kBl[3], 1, 0};
+    Plan best{kBl[3], 1, 0, 0};
     double best_cost = 1e30;
     for (const TileCfg& t : kBl) {
         const int bit = t.bk == 16 ? 1 : t.bk == 32 ? 2 : 4;
@@ -2283,10 +2322,10 @@ bool plan_bl(const GemmParams& p, int nbatch, int blm, const shp::GemmTune& tn, 
             int real = (p.K + kps - 1) / kps;
             // the model keeps 128 K per split; a forced split count may go down to one K tile
             if (s > 1 && (real != s || kps < (tn.splits ? kq : 128))) continue;
-            double c = plan_cost(p, nbatch, t, s, kps);
+            double c = bl_plan_cost(p, nbatch, amode, t, s, kps);
             if (c < best_cost * 0.97) {
                 best_cost = c;
-                best = Plan{t, s, kps};
+                best = Plan{t, s, kps, c};
             }
         }
     }
@@ -2305,11 +2344,11 @@ Plan plan_gemm(const GemmParams& p, int nbatch, bool hot, bool dma_ok, bool conv
         tuned_plan(p, nbatch, amode, bmode, hot, blm, &tuned))
         return tuned;
     if (blm && tn.bl >= 0 && (tn.bl > 0 || (tn.dma <= 0 && !tn.pg)) &&
-        plan_bl(p, nbatch, blm, tn, &tuned))
+        plan_bl(p, nbatch, amode, blm, tn, &tuned))
         return tuned;
     if (dma_ok && conv_a && tn.dma == 0 && !tn.splits && dma_preferred(p, nbatch))
-        return Plan{{128, 64, 16, true}, 1, ((p.K + 31) / 32) * 32};
-    Plan best{{128, 128, 32, false}, 1, 0};
+        return Plan{{128, 64, 16, true}, 1, ((p.K + 31) / 32) * 32, 0};
+    Plan best{{128, 128, 32, false}, 1, 0, 0};
     double best_cost = 1e30;
     for (int ti = 0; ti < 5; ++ti) {
         const bool dma = ti >= 3;
@@ -2331,7 +2370,7 @@ Plan plan_gemm(const GemmParams& p, int nbatch, bool hot, bool dma_ok, bool conv
                 double c = plan_cost(p, nbatch, t, s, kps);
                 if (c < best_cost * 0.97) {  // prefer the earlier (simpler) plan on near ties
                     best_cost = c;
-                    best = Plan{t, s, kps};
+                    best = Plan{t, s, kps, 0};
                 }
             }
         }
@@ -2512,13 +2551,16 @@ int gemm_launch(hipStream_t stream, GemmParams p, int amode, int bmode, int cmod
         const int v = smallk_variant(p, amode, bmode, cmode, nbatch);
         if (v) return launch_smallk(stream, p, amode, v);
     }
-    if (direct_eligible(p, amode, bmode, cmode)) {
+    const bool direct_ok = direct_eligible(p, amode, bmode, cmode);
+    if (direct_ok) {
         const int ds = direct_splits(p, direct_tune(tn));
         if (ds == 1 || (ds > 1 && workspace && workspace_bytes >= direct_workspace(p, ds)))
             return direct_launch(stream, p, amode, bmode, ds, workspace);
     }
     const int blm = bl_mask(p, amode, bmode, cmode);
     Plan pl = plan_gemm(p, nbatch, hot, dma_ok, amode == A_CONV_NHWC4, tn, amode, bmode, blm);
+    if (direct_ok && direct_tune(tn) == 0 && direct_cost(p, amode) < pl.cost)
+        return direct_launch(stream, p, amode, bmode, 1, workspace);
     size_t need = pl.splits > 1
                       ? kSplitCounterBytes + (size_t)pl.splits * nbatch * p.M * p.N * sizeof(float)
                       : 0;

@@ -259,7 +259,8 @@ bool direct_eligible(const GemmParams& p, int amode, int bmode, int cmode) {
 // always, with that many splits).  The line lies at one workgroup per CU: with at most 256 tiles
 // the direct kernel won on all 114 of the swept shapes (1x1 and 3x3 convolutions of CNN layers at
 // batches 1-32, BERT's and TinyLlama's products with 1-2,048 rows) by 1.08-1.82 times, 1.35 at the
-// median (512x768x768 16.3 -> 10.4 us); above it the tiled kernels did on 57 of 80.  K is split while every CU
+// median (512x768x768 16.3 -> 10.4 us); above it the tiled kernels did on 57 of 80, and gemm_launch
+// compares both estimates.  K is split while every CU
 // still gets at most one workgroup and a split keeps 128 k: a second round of workgroups costs more
 // than the shorter chains give (200x2304x768, 252 tiles: 10.5 us unsplit, 13.2 in two).
 int direct_splits(const GemmParams& p, int tune) {

@@ -1129,6 +1129,29 @@ def test_gemm_direct_convolutions(ctx, orc, n, ih, ic, k, oc, s):
             ctx.tune("gemm_small", 0)
 
 
+@pytest.mark.parametrize("m,k,n", [(384, 768, 3072), (515, 2048, 1300), (1071, 1280, 500), (1600, 80, 772)])
+def test_gemm_planned_products(ctx, orc, m, k, n):
+    """More tiles than CUs, where the plan goes by estimated time: the direct kernel over two and
+    three rounds of workgroups, tiled kernels with and without K splits, row and column tails."""
+    x, w, b, r = rnd(m, k), rnd(k, n), rnd(n), rnd(m, n)
+    for res in (None, r):
+        y, ref = both(ctx, orc, "hlo_dot_rank2", x, w, m * n, [m, k, n, m * n], bias=b, residual=res, act="relu")
+        # k products of magnitude ~1 sum in fp32: the error grows as sqrt(k) eps sqrt(k)
+        assert_close(y, ref, 1e-4, 4 * k * 6e-8, f"planned {m}x{n}x{k}")
+
+
+@pytest.mark.parametrize("n,ih,ic,k,oc,s", [(8, 28, 128, 3, 128, 1), (9, 15, 96, 3, 196, 1), (5, 33, 80, 5, 100, 2)])
+def test_gemm_planned_convolutions(ctx, orc, n, ih, ic, k, oc, s):
+    """The same on convolutions with taps."""
+    p = (k - 1) // 2
+    oh = (ih + 2 * p - k) // s + 1
+    x, w = rnd(n, ih, ih, ic), rnd(k, k, ic, oc) * np.float32(np.sqrt(2.0 / (k * k * ic)))
+    total = n * oh * oh * oc
+    push = [n, ih, ih, ic, k, k, oc, oh, oh, s, s, p, p, total]
+    y, ref = both(ctx, orc, "hlo_conv_nhwc_hwio", x, w, total, push, bias=rnd(oc), act="relu6")
+    assert_close(y, ref, 1e-4, 1e-4, f"planned conv {n}x{ih} {ic}->{oc} k{k}")
+
+
 @pytest.mark.parametrize("n", [1, 3, 1000, 131073, 262143, 262144, 262145, 300001, (16 << 20) + 5])
 def test_run_kernel_sizes(n):
     """Host buffers in and out around the pinned-staging (1 MiB each way) and kept-buffer (64 MiB)
