@@ -749,10 +749,10 @@ const TunedBlock* tuned_block(const IrShape& sh) {
 //   4x28x28x32 to 64: 17.5 against 13.7);
 // * beyond, where the launches are latencies: 3x3, ce under 900, cin * pixels up to 37,000
 //   (1x14x14x96: 14.0 against 14.7; 4x14x14x96: 22.1 against 18.8; 12x7x7x192: 63.2 against 27.9).
-// The depthwise + projection form (no expand) pays with ce <= 96 at any size; at stride 1 up to ce
-// 256 (24x56x56x144: 0.87 of the two launches) and up to ce 700 while the projection is small
-// (4x14x14x384: 0.95, 12x14x14x384: 1.15); at stride 2 up to ce 256 for few outputs, more of them
-// with a 5x5 window, whose taps the fused form reads from LDS.
+// The depthwise + projection form (no expand) pays with ce <= 96 on maps of 56x56 and more, the
+// only ones measured; at stride 1 up to ce 256 (24x56x56x144: 0.87 of the two launches) and up to
+// ce 700 while the projection is small (4x14x14x384: 0.95, 12x14x14x384: 1.15); at stride 2 up to
+// ce 256 for few outputs, more of them with a 5x5 window, whose taps the fused form reads from LDS.
 bool fusion_pays(const IrShape& sh) {
     if (const TunedBlock* t = tuned_block(sh)) return t->fuse;
     const int64_t in = (int64_t)sh.n * sh.h * sh.w, out = (int64_t)sh.n * sh.oh * sh.ow;
@@ -761,7 +761,7 @@ bool fusion_pays(const IrShape& sh) {
         if (sh.cin <= 48) return in <= 2000;
         return sh.k == 3 && sh.ce < 900 && sh.cin * in <= 37000;
     }
-    if (sh.ce <= 96) return true;
+    if (sh.ce <= 96) return out >= 3000;
     if (sh.s == 1)
         return sh.ce <= 256 || (sh.ce <= 480 && out <= (sh.k == 5 ? 1600 : 1200)) ||
                (sh.ce <= 700 && out <= 800);
