@@ -61,6 +61,10 @@ struct GemmParams {
 // launch leaves them zero again.  The partials follow.
 constexpr size_t kSplitCounterBytes = 65536;
 
+// Largest split-K workspace (counters + partials) of one shp_launch_static launch.  The
+// ResNet-50 b32 convolutions need at most 18.4 MiB, the BERT-base b8 s128 dots 36 MiB.
+constexpr size_t kStaticScratchBytes = size_t(64) << 20;
+
 // Launch C = epilogue(A*B) for the problem; picks tile shape and split-K (`tune` may force
 // parts of that choice, or be null).  `workspace`/`workspace_bytes` provide the split-K
 // partials (may be null: no split).

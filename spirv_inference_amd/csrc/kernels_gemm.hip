@@ -2322,6 +2322,12 @@ bool plan_bl(const GemmParams& p, int nbatch, int amode, int blm, const shp::Gem
             int real = (p.K + kps - 1) / kps;
             // the model keeps 128 K per split; a forced split count may go down to one K tile
             if (s > 1 && (real != s || kps < (tn.splits ? kq : 128))) continue;
+            // splits that would not fit shp_launch_static's scratch: a convolution of that size has
+            // tiles enough without them
+            if (s > 1 && !tn.splits && amode == shp::A_CONV_NHWC4 &&
+                shp::kSplitCounterBytes + (size_t)s * nbatch * p.M * p.N * sizeof(float) >
+                    shp::kStaticScratchBytes)
+                continue;
             double c = bl_plan_cost(p, nbatch, amode, t, s, kps);
             if (c < best_cost * 0.97) {
                 best_cost = c;

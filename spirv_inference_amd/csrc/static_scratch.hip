@@ -15,12 +15,6 @@
 #include "gemm.h"
 #include "runtime.h"
 
-namespace shp {
-// Largest split-K workspace one launch may use: counters (kSplitCounterBytes) + partials.
-// The ResNet-50 b32 convolutions need at most 18.4 MiB, the BERT-base b8 s128 dots 36 MiB.
-constexpr size_t kStaticScratchBytes = size_t(64) << 20;
-}  // namespace shp
-
 // The array itself.  In host code `scratch` names a host-side stand-in, never the device
 // memory: host code uses the per-device address from hipGetSymbolAddress instead.
 static __device__ __align__(256) float scratch[shp::kStaticScratchBytes / sizeof(float)];
