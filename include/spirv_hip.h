@@ -240,9 +240,10 @@ int shp_llama_step(shp_llama* lm, int32_t token);
 int shp_llama_decode(shp_llama* lm, int32_t n_steps);
 /* Synchronises and copies the argmax of every step so far (one per step, in order). */
 int shp_llama_tokens(shp_llama* lm, int32_t* out, int32_t cap, int32_t* n_out);
-/* Feeds prompt[0..n_prompt) (all positions of up to 512 in one pass over the weights, on any
- * engine) then generates n_new greedy tokens into out_tokens (synchronous).  Stops early at token 2 (EOS) or 0 (PAD) like run_llama_spirv.py:292-294;
- * returns the number written through *n_out. */
+/* Feeds prompt[0..n_prompt) (from three ids on, all positions of up to 512 in one pass over the
+ * weights, on any engine) then generates n_new greedy tokens into out_tokens (synchronous).
+ * Stops early at token 2 (EOS) or 0 (PAD) like run_llama_spirv.py:292-294; returns the number
+ * written through *n_out. */
 int shp_llama_generate(shp_llama* lm, const int32_t* prompt, int32_t n_prompt, int32_t n_new,
                        int32_t* out_tokens, int32_t* n_out);
 int shp_llama_use_graph(shp_llama* lm, int enable);
