@@ -722,20 +722,21 @@ __device__ __forceinline__ void stage_copy(const float* __restrict__ s, float* _
 
 __global__ __launch_bounds__(kBlock) void host_stage_kernel(const float* __restrict__ p0,
                                                             const float* __restrict__ p1, float* d0,
-                                                            size_t n0, float* d1, size_t n1,
-                                                            float* d2, size_t n2) {
+                                                            size_t n0, size_t e0, float* d1,
+                                                            size_t n1, size_t e1, float* d2,
+                                                            size_t n2) {
     const size_t tid = (size_t)blockIdx.x * kBlock + threadIdx.x;
     const size_t stride = (size_t)gridDim.x * kBlock;
-    stage_copy(p0, d0, n0, tid, stride);
-    stage_copy(p1, d1, n1, tid, stride);
+    if (p0) {
+        stage_copy(p0, d0, n0, tid, stride);
+        stage_copy(p1, d1, n1, tid, stride);
+    }
+    for (size_t i = n0 + tid; i < e0; i += stride) d0[i] = 0.0f;
+    for (size_t i = n1 + tid; i < e1; i += stride) d1[i] = 0.0f;
     for (size_t i = tid; i < n2 / 4; i += stride)
         reinterpret_cast<ew4*>(d2)[i] = ew4{0.f, 0.f, 0.f, 0.f};
     for (size_t i = n2 / 4 * 4 + tid; i < n2; i += stride) d2[i] = 0.0f;
-    if (tid == 0) {  // an unused binding holds one zero
-        if (!n0) d0[0] = 0.0f;
-        if (!n1) d1[0] = 0.0f;
-        if (!n2) d2[0] = 0.0f;
-    }
+    if (tid == 0 && !n2) d2[0] = 0.0f;  // an unused binding holds one zero
 }
 
 __global__ __launch_bounds__(kBlock) void host_fetch_kernel(const float* __restrict__ d,
@@ -778,10 +779,10 @@ __global__ __launch_bounds__(kBlock) void fill_random_kernel(float* __restrict__
 namespace shp {
 
 int host_stage_launch(hipStream_t s, const float* p0, const float* p1, float* d0, size_t n0,
-                      float* d1, size_t n1, float* d2, size_t n2) {
-    const size_t most = std::max(std::max(n0, n1), n2);
+                      size_t e0, float* d1, size_t n1, size_t e1, float* d2, size_t n2) {
+    const size_t most = std::max({n0, e0, n1, e1, n2});
     hipLaunchKernelGGL(host_stage_kernel, dim3(ew_grid(most / 4 + 1)), dim3(kBlock), 0, s, p0, p1,
-                       d0, n0, d1, n1, d2, n2);
+                       d0, n0, e0, d1, n1, e1, d2, n2);
     SHP_HIP_CHECK(hipGetLastError());
     return SHP_OK;
 }

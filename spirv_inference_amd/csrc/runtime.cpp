@@ -152,6 +152,7 @@ int Ctx::io_buffer(int i, size_t bytes) {
     io_bytes[i] = 0;
     SHP_HIP_CHECK(hipMalloc(&io[i], cap));
     io_bytes[i] = cap;
+    io_used_floats[i] = cap / 4;  // of unknown content
     return SHP_OK;
 }
 
@@ -428,6 +429,15 @@ int shp_launch_ex(shp_ctx* ctx, const char* kernel, const void* in0, const void*
                                                epi);
 }
 
+// Floats of the additive mask a kernel reads from in1 where one is given (it takes null for none), 0
+// for kernels whose in1 is not optional.
+static size_t optional_mask_floats(const char* kernel, const int32_t* push, size_t n_push) {
+    if (!std::strcmp(kernel, "softmax_rows")) return n_push >= 2 && push[1] > 0 ? push[1] : 0;
+    if (!std::strcmp(kernel, "attention_fused") || !std::strcmp(kernel, "attention_rows"))
+        return n_push >= 3 && push[2] > 0 ? push[2] : 0;
+    return 0;
+}
+
 int shp_run_kernel(shp_ctx* ctx, const char* kernel, const float* in0, size_t n0,
                    const float* in1, size_t n1, float* out, size_t n_out, const int32_t* push,
                    size_t n_push, uint32_t grid_hint, shp_run_info* info) {
@@ -449,8 +459,12 @@ int shp_run_kernel(shp_ctx* ctx, const char* kernel, const float* in0, size_t n0
     // call: 80 us for 1,000 floats, 27 us now); past kIoKeep bytes one is given back after the call.
     // Up to kIoStage bytes each way go through pinned memory and one kernel (4 KB there and back:
     // 26 us against 29 for two pageable copies, 512 KB: 62 against 65); above that the runtime's own
-    // copies are as fast.
-    const size_t b0 = (n0 ? n0 : 1) * 4, b1 = (n1 ? n1 : 1) * 4, b2 = (n_out ? n_out : 1) * 4;
+    // copies are as fast.  What an earlier call left behind a shorter input is zeroed, so a kernel that
+    // reads past the input it was given (an additive mask given as the one zero of an unused binding)
+    // never sees another call's data; a mask given as no elements at all is no mask.
+    const size_t mask = std::min(optional_mask_floats(kernel, push, n_push), n0);
+    const size_t b0 = (n0 ? n0 : 1) * 4, b2 = (n_out ? n_out : 1) * 4;
+    const size_t b1 = std::max<size_t>(n1 ? std::max(n1, mask) : 1, 1) * 4;
     int rc = c->io_prepare();
     if (!rc) rc = c->io_buffer(0, b0);
     if (!rc) rc = c->io_buffer(1, b1);
@@ -461,16 +475,20 @@ int shp_run_kernel(shp_ctx* ctx, const char* kernel, const float* in0, size_t n0
     const bool down = c->stage_down && n_out * 4 <= Ctx::kIoStage;
     do {
         if (rc) break;
+        // zeroed behind each input: up to what an earlier call wrote, at least one element of an
+        // unused binding
+        const size_t e0 = std::max<size_t>(c->io_used_floats[0], 1);
+        const size_t e1 = std::max<size_t>(c->io_used_floats[1], 1);
         if (up) {
             if (n0) std::memcpy(c->stage_up, in0, n0 * 4);
             if (n1) std::memcpy(c->stage_up + off1, in1, n1 * 4);
             rc = shp::host_stage_launch(c->stream, (const float*)c->stage_up,
-                                        (const float*)(c->stage_up + off1), d0, n0, d1, n1, d2,
-                                        n_out);
+                                        (const float*)(c->stage_up + off1), d0, n0, e0, d1, n1, e1,
+                                        d2, n_out);
             if (rc) break;
         } else {
-            // zeroes the output and the first element of an unused binding
-            rc = shp::host_stage_launch(c->stream, nullptr, nullptr, d0, 0, d1, 0, d2, n_out);
+            rc = shp::host_stage_launch(c->stream, nullptr, nullptr, d0, n0, e0, d1, n1, e1, d2,
+                                        n_out);
             if (rc) break;
             if (n0 && hipMemcpyAsync(d0, in0, n0 * 4, hipMemcpyHostToDevice, c->stream) != hipSuccess) {
                 rc = fail(SHP_ERR_HIP, "shp_run_kernel: upload in0 failed");
@@ -481,8 +499,10 @@ int shp_run_kernel(shp_ctx* ctx, const char* kernel, const float* in0, size_t n0
                 break;
             }
         }
+        c->io_used_floats[0] = n0;
+        c->io_used_floats[1] = n1;
         (void)hipEventRecord(c->io_events[0], c->stream);
-        rc = c->launch(kernel, d0, d1, d2, push, n_push, n_out, nullptr);
+        rc = c->launch(kernel, d0, mask && !n1 ? nullptr : d1, d2, push, n_push, n_out, nullptr);
         if (rc) break;
         (void)hipEventRecord(c->io_events[1], c->stream);
         if (n_out && down) {

@@ -30,6 +30,7 @@ struct Ctx {
     static constexpr size_t kIoKeep = 64u << 20, kIoStage = 1u << 20;
     void* io[3] = {nullptr, nullptr, nullptr};
     size_t io_bytes[3] = {0, 0, 0};
+    size_t io_used_floats[3] = {0, 0, 0};  // inputs: floats from here on are zero
     char *stage_up = nullptr, *stage_down = nullptr;
     hipEvent_t io_events[2] = {nullptr, nullptr};
     bool io_used = false;
@@ -61,10 +62,11 @@ struct Ctx {
 // a memset or copy node into the caller's graph or breaking the capture.
 int refuse_while_capturing(hipStream_t stream, const char* what);
 
-// shp_run_kernel's bindings, uploaded from pinned memory (both device-visible; n0 or n1 may be 0)
-// with the output zeroed, and the output downloaded to it: one kernel each way.
+// shp_run_kernel's bindings, uploaded from pinned memory (n0 or n1 floats, which may be 0; none where
+// pinned0 is null) and zeroed from there up to e0 and e1, with the output zeroed; and the output
+// downloaded to it: one kernel each way.
 int host_stage_launch(hipStream_t s, const float* pinned0, const float* pinned1, float* d0,
-                      size_t n0, float* d1, size_t n1, float* d2, size_t n2);
+                      size_t n0, size_t e0, float* d1, size_t n1, size_t e1, float* d2, size_t n2);
 int host_fetch_launch(hipStream_t s, const float* d2, float* pinned, size_t n2);
 
 // Resolves, once per device and with that device current, the device address of the fixed

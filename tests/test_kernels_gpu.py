@@ -1170,6 +1170,30 @@ def test_run_kernel_sizes(n):
             assert out.elapsed_ms > 0
 
 
+@pytest.mark.parametrize("mask", ["none", "one zero", "short", "full"])
+@pytest.mark.parametrize("before", [1000, 300000])
+def test_run_kernel_mask_is_the_calls_own(ctx, orc, mask, before):
+    """A kernel with an optional mask (in1) sees this call's mask, padded with zeros where it is short,
+    or none: never what an earlier call of the context left in the binding."""
+    from spirv_inference_amd import KernelRun
+    cols, S, B, H = 500, 40, 2, 3
+    x, qkv = rnd(7, cols), rnd(B * S * 3 * H * 64)
+    sb = int(np.array([0.5], np.float32).view(np.int32)[0])
+    att = [B, H, S, 64, 3 * H * 64, 0, H * 64, 2 * H * 64, H * 64, sb, B * S * H * 64]
+    for kernel, a, push, n, width in (("softmax_rows", x, [7, cols, sb], x.size, cols),
+                                      ("attention_rows", qkv, att, att[10], S)):
+        given = {"none": np.zeros(0, np.float32), "one zero": np.zeros(1, np.float32),
+                 "short": rnd(width // 2), "full": rnd(width)}[mask]
+        padded = np.zeros(width, np.float32)
+        padded[:given.size] = given
+        for _ in range(2):
+            y = np.abs(rnd(before)) * 50
+            ctx.run_kernel(KernelRun("add", "add", y, y, before, 1, [before]))
+            got = ctx.run_kernel(KernelRun(kernel, kernel, a, given, n, 1, push)).values
+            want = orc.run(kernel, a, padded, n, push)
+            assert_close(got, want, 1e-4, 1e-4, f"{kernel}, mask {mask}, after add of {before}")
+
+
 def test_run_kernel_output_starts_at_zero(ctx):
     """A kernel that writes part of its output leaves zeros in the rest, whatever ran before."""
     from spirv_inference_amd import KernelRun
