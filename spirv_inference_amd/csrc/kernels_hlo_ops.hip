@@ -644,8 +644,9 @@ __global__ __launch_bounds__(256) void reduce_rows_kernel(const float* __restric
     const int cols = kRedTile / rows, ls = cols + 4;
     const int64_t r0 = (int64_t)blockIdx.x * rows;
     // Load i of a thread is a fixed distance from its load 0: a tile row is cols / W loads, a
-    // power of two, so 256 threads cover whole rows or a part of one.  No bounds checks: rows past
-    // the end are outside the buffer range, columns past n are never folded.
+    // power of two, so 256 threads cover whole rows or a part of one.  The buffer range is the
+    // check: rows past the end lie outside it (the whole distance is in the vector offset, which is
+    // what the range bounds), columns past n are another row's or outside, and never folded.
     const int cw = cols / W, sh = 31 - __clz(cw);
     const __amdgpu_buffer_rsrc_t xr = buffer_rsrc(x + r0 * n, min((int64_t)rows, nrows - r0) * n);
     const int row = cw < 256 ? tid >> sh : 0, col = (cw < 256 ? tid & (cw - 1) : tid) * W;
@@ -657,12 +658,12 @@ __global__ __launch_bounds__(256) void reduce_rows_kernel(const float* __restric
         for (int i = 0; i < NL; ++i) {
             const int di = cw < 256 ? i * (256 >> sh) : (i * 256) >> sh;  // rows from load 0
             const int dc = cw < 256 ? 0 : ((i * 256) & (cw - 1)) * W;
-            const unsigned so = (unsigned)(di * n + dc + c0) * 4u;
+            const unsigned off = voff + (unsigned)(di * n + dc + c0) * 4u;
             if constexpr (VEC) {
-                const f4v v = __builtin_bit_cast(f4v, __builtin_amdgcn_raw_buffer_load_b128(xr, voff, so, 0));
+                const f4v v = __builtin_bit_cast(f4v, __builtin_amdgcn_raw_buffer_load_b128(xr, off, 0, 0));
                 st[i][0] = v.x; st[i][1] = v.y; st[i][2] = v.z; st[i][3] = v.w;
             } else {
-                st[i][0] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(xr, voff, so, 0));
+                st[i][0] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(xr, off, 0, 0));
             }
         }
     };

@@ -1001,6 +1001,18 @@ def test_hlo_reduce(ctx, orc, shape, dims):
                                       orc.run("hlo_reduce", x, None, kept, push))
 
 
+@pytest.mark.parametrize("rows,n", [(1, 4 << 20), (1, (4 << 20) + 3), (3, 1 << 20), (257, 4100), (1025, 768)])
+def test_hlo_reduce_few_long_rows(ctx, orc, rows, n):
+    """Fewer rows than a workgroup's tile holds, at the end of an allocation: the tile's other rows lie
+    up to three tensors past it and must not be loaded."""
+    from spirv_inference_amd import hlo_ops as H
+    x = rnd(rows, n)
+    for kind, init in (("sum", 0.0), ("max", -np.inf)):
+        push = H.reduce_push(kind, (rows, n), (1,), init)
+        np.testing.assert_array_equal(_dev(ctx, "hlo_reduce", x, None, rows, push),
+                                      orc.run("hlo_reduce", x, None, rows, push))
+
+
 @pytest.mark.parametrize("cols", [1, 3, 4, 63, 64, 100, 255, 256, 260, 511, 768, 1001, 1024, 1028, 2047, 2048, 2052, 3001])
 @pytest.mark.parametrize("rows", [1, 5, 130])
 def test_row_kernels_all_widths(ctx, orc, rows, cols):
