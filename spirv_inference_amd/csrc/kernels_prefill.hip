@@ -73,9 +73,9 @@ __global__ __launch_bounds__(kSkWaves * 64, MT <= 2 ? 4 : 2) void skinny_kernel(
     Set st[ST];
     auto load = [&](int s, Set& d) __attribute__((always_inline)) {
         // K % 4 == 0, so a lane's 16 bytes lie on one side of the end; past it (also the steps
-        // beyond ns) nothing is read
+        // beyond ns) nothing is read: the vector offset is past every range, the scalar one never
         const bool in = s < ns && k0 + 16 * s < ke;
-        const unsigned so = (unsigned)(s * 64);
+        const unsigned so = s < ns ? (unsigned)(s * 64) : 0u;
 #pragma unroll
         for (int i = 0; i < NT; ++i)
             d.w[i] = __builtin_bit_cast(

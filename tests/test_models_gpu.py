@@ -346,6 +346,25 @@ def test_llama_prompt_pass_equals_token_steps(ctx, n):
             assert_close(got[k].ravel(), w.ravel(), 1e-4, 1e-4, f"prompt of {n}: {k}")
 
 
+@pytest.mark.parametrize("hidden,ffn,vocab", [(8, 4, 8), (16, 12, 24), (72, 20, 40)])
+@pytest.mark.parametrize("n", [3, 20])
+def test_llama_prompt_pass_of_narrow_models(ctx, hidden, ffn, vocab, n):
+    """Products whose K is shorter than the steps the prompt kernels load ahead: no load past the
+    operands, and the same as the prompt fed id by id."""
+    from spirv_inference_amd.models import Llama
+    cfg = dict(SMALL, hidden=hidden, n_heads=2, n_kv_heads=1, ffn=ffn, vocab=vocab)
+    prompt = [int(t) for t in np.random.default_rng(n).integers(3, vocab, n)]
+    with Llama(ctx, seed=9, **cfg) as lm:
+        lm.reset()
+        for t in prompt:
+            lm.step(t)
+        ctx.sync()
+        tokens, want = lm.tokens(), lm.logits()
+        lm.generate(prompt, 1)
+        assert lm.tokens() == tokens
+        assert_close(lm.logits(), want, 1e-5, 1e-4, f"hidden {hidden}, prompt of {n}")
+
+
 def test_llama_generate_refuses_bad_prompts(ctx):
     from spirv_inference_amd import ShpError
     from spirv_inference_amd.models import Llama
