@@ -2322,9 +2322,9 @@ bool plan_bl(const GemmParams& p, int nbatch, int amode, int blm, const shp::Gem
             int real = (p.K + kps - 1) / kps;
             // the model keeps 128 K per split; a forced split count may go down to one K tile
             if (s > 1 && (real != s || kps < (tn.splits ? kq : 128))) continue;
-            // splits that would not fit shp_launch_static's scratch: a convolution of that size has
-            // tiles enough without them
-            if (s > 1 && !tn.splits && amode == shp::A_CONV_NHWC4 &&
+            // splits that would not fit shp_launch_static's scratch: an output of that size has tiles
+            // enough without them (448x11008x11008 859 -> 873 us, 4096x1024x16384 1.028 -> 1.031 ms)
+            if (s > 1 && !tn.splits &&
                 shp::kSplitCounterBytes + (size_t)s * nbatch * p.M * p.N * sizeof(float) >
                     shp::kStaticScratchBytes)
                 continue;

@@ -68,6 +68,30 @@ def test_static_scratch_matches_workspace_launch_twice():
         assert _workspace_bytes(ctx_static) == 0
 
 
+@pytest.mark.parametrize("kernel,m,k,n", [("hlo_dot_rank2", 4608, 8192, 1280), ("hlo_dot_rank2", 2848, 11008, 2048),
+                                          ("hlo_dot_rank2", 448, 11008, 11008),
+                                          ("fully_connected", 5760, 8192, 1024),
+                                          ("dot_general_strided", 768, 12288, 4608)])
+def test_static_scratch_holds_deep_products(kernel, m, k, n):
+    """Products of many tiles and a deep K are planned with splits that the static scratch holds."""
+    with Context("any") as ctx_static, Context("any") as ctx_ws:
+        got = []
+        for ctx, launch in ((ctx_static, lib().shp_launch_static), (ctx_ws, lib().shp_launch_ex)):
+            a = ctx.fill_random(ctx.empty(m * k), 31, 1)
+            b = ctx.fill_random(ctx.empty(k * n + n), 31, 2)
+            c = ctx.empty(m * n)
+            push = {"hlo_dot_rank2": [m, k, n, m * n], "fully_connected": [m, k, n, m * n],
+                    "dot_general_strided": [1, 1, m, n, k, 0, 0, k, 1, 0, 0, 1, k, 0, 0, n, 1]}[kernel]
+            arr = (C.c_int32 * len(push))(*push)
+            check(launch(ctx.handle, kernel.encode(), a.ptr, b.ptr, c.ptr, arr, len(push), m * n, None), kernel)
+            ctx.sync()
+            got.append(c.download())
+            for t in (a, b, c):
+                t.free()
+        assert np.isfinite(got[0]).all() and np.array_equal(*got)
+        assert _workspace_bytes(ctx_static) == 0
+
+
 def test_static_scratch_rejects_plans_beyond_its_size():
     """A dot whose plan wants 64.06 MiB of split-K scratch is refused before any launch."""
     m, k, n = 4096, 16384, 1024
