@@ -666,7 +666,7 @@ int launch_bias_act(const shp::Launch& l) {
         const unsigned n4 = (unsigned)(l.out_elems / 4);
         const bool many = n4 >= kManyVec;
         hipLaunchKernelGGL((many ? bias_act4_kernel<4> : bias_act4_kernel<1>),
-                           dim3(many ? ew_grid_vec(n4) : (n4 + kBlock - 1) / kBlock), dim3(kBlock), 0, l.stream,
+                           dim3(many ? ew_grid_vec(n4) : shp::grid_1d(n4, kBlock)), dim3(kBlock), 0, l.stream,
                            (const ew4*)l.in0, (ew4*)l.out, n4, shpd::fast_div(l.push[1] / 4),
                            (const ew4*)l.epi->bias, (const ew4*)l.epi->residual, l.epi->act,
                            l.epi->alpha);

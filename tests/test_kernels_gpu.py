@@ -1082,6 +1082,16 @@ def test_bias_act_forms(ctx, orc, n, c, act):
         assert_close(y, r, 1e-5, 1e-5, f"bias_act {n} {c} {act}")
 
 
+def test_bias_act_of_nothing(ctx):
+    """An empty tensor is a valid call that does nothing."""
+    x, b = ctx.tensor(rnd(8)), ctx.tensor(rnd(8))
+    for c in (8, 7):
+        ctx.launch("bias_act", x, None, x, [0, c], out_elems=0, bias=b, act="relu")
+    ctx.sync()
+    for t in (x, b):
+        t.free()
+
+
 def test_hlo_shape_ops_fail_closed(ctx):
     from spirv_inference_amd import hlo_ops as H
     with pytest.raises(RuntimeError):  # not a permutation
