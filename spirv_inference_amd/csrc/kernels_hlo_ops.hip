@@ -94,7 +94,7 @@ int read_dims(const int32_t* q, int r, int* dims, const char* kernel) {
 //   elements where length or alignment do not allow 16 bytes;
 // * a transpose (some other axis is the contiguous one): tiles of both axes through LDS, so reads run
 //   along the source's contiguous axis and writes along the output's (8x306x32x64 to 8x32x64x306:
-//   31 -> 12 us).
+//   31 -> 12 us); single elements where the matrices or the tensor are small.
 using shpd::FastDiv;
 using shpd::fast_div;
 using shpd::fdiv;
@@ -254,14 +254,21 @@ int launch_gather(const shp::Launch& l, const Gather& g0) {
         int bx = -1;  // the source's contiguous axis
         for (int k = 0; k < r - 1; ++k)
             if (st[k] == 1) bx = k;
-        if (bx >= 0 && st[r - 1] > 1 && d[bx] >= 8 && n >= 4) {
-            Tiles p{};
+        Tiles p{};
+        if (bx >= 0 && st[r - 1] > 1) {
             p.a = n;
             p.b = d[bx];
             // up to 64 of each, or one axis longer where the other is short
             p.ta = std::min(n, 64);
             p.tb = std::min(p.b, std::min(256, 4096 / p.ta));
             p.ta = std::min(n, std::min(256, 4096 / p.tb));
+        }
+        // A tile pays a load, LDS and store latency of its own: it wins from 1,024 elements a tile on
+        // (200,000 matrices of 32x32 329 us, 606 as single elements, but of 16x32 235 against 212 and of
+        // 4x8 134 against 11), once there are 1.25 M elements, which fill the GPU with tiles (8x384x7x64
+        // 7.8 against 10.7; 256 matrices of 64x64 6.6 against 4.9, one 300x33 5.8 against 2.6).  So a
+        // launch has fewer than 2^24 tiles.
+        if (p.ta * p.tb >= 1024 && l.out_elems >= (5u << 18)) {
             p.sa = st[r - 1];
             p.base = g.base;
             p.fta = fast_div(p.ta);

@@ -1034,7 +1034,13 @@ def test_row_kernels_all_widths(ctx, orc, rows, cols):
 GATHERS = [((3, 5, 7, 64), (0, 2, 1, 3)), ((3, 5, 7, 33), (0, 2, 1, 3)), ((2, 70, 12, 64), (0, 2, 3, 1)),
            ((2, 70, 12, 33), (0, 3, 2, 1)), ((1, 300, 4, 64), (0, 1, 3, 2)), ((7, 9, 130, 3), (2, 0, 1, 3)),
            ((65, 129), (1, 0)), ((300, 5), (1, 0)), ((5, 300), (1, 0)), ((2, 3, 2, 5, 3, 4), (5, 0, 3, 1, 4, 2)),
-           ((64, 64, 1, 16), (3, 2, 1, 0)), ((8,), (0,)), ((1, 1), (1, 0)), ((4, 257, 66), (2, 1, 0))]
+           ((64, 64, 1, 16), (3, 2, 1, 0)), ((8,), (0,)), ((1, 1), (1, 0)), ((4, 257, 66), (2, 1, 0)),
+           # from 1.25 M elements on: tiles of 1,024 elements and more, whole and ragged, of few and of
+           # many matrices; single elements and 16-byte rows above four a thread (2^20 of them)
+           ((1103, 1201), (1, 0)), ((40, 33, 1031), (0, 2, 1)), ((5, 301, 12, 77), (0, 2, 3, 1)),
+           ((2, 700, 31, 33), (0, 3, 2, 1)), ((701, 45, 47), (0, 2, 1)), ((1300, 32, 32), (0, 2, 1)),
+           ((1301, 31, 33), (2, 0, 1)), ((30011, 7, 9), (0, 2, 1)), ((41000, 8, 4), (0, 2, 1)),
+           ((3, 311, 9, 157), (0, 2, 1, 3)), ((4, 1030, 17, 64), (0, 2, 1, 3))]
 
 
 @pytest.mark.parametrize("shape,perm", GATHERS)
@@ -1053,6 +1059,22 @@ def test_gather_forms_transpose(ctx, orc, shape, perm):
     ctx.sync()
     np.testing.assert_array_equal(out.download()[1:], want)
     for t in (big, out):
+        t.free()
+
+
+def test_gather_of_very_many_small_matrices(ctx):
+    """[2^24, 4, 8] transposed to [2^24, 8, 4]: as many matrices as no launch could have workgroups for."""
+    from spirv_inference_amd import hlo_ops as H
+    from spirv_inference_amd.runtime import DeviceTensor
+    N = 1 << 24
+    x, y = ctx.empty(N * 32), ctx.empty(N * 32)
+    ctx.fill_random(x, 3, 1)
+    ctx.launch("hlo_transpose", x, None, y, H.transpose_push((N, 4, 8), (0, 2, 1)))
+    ctx.sync()
+    for at in (0, N // 2 + 5, N - 300):
+        part = lambda t: DeviceTensor(ctx, 300 * 32, ptr=t.ptr + at * 128, owned=False).download()
+        np.testing.assert_array_equal(part(y).reshape(300, 8, 4), part(x).reshape(300, 4, 8).transpose(0, 2, 1))
+    for t in (x, y):
         t.free()
 
 
