@@ -841,28 +841,33 @@ int launch_reduce_nd(const shp::Launch& l) {
     rc = shp::check_total(l, q[2], "hlo_reduce");
     if (rc) return rc;
     // One reduced run: rows of contiguous elements go through LDS tiles (the fewest rows per
-    // workgroup that still give every CU one).  So do columns up to 65,536 outputs, a wavefront
-    // per SIMD if each had a thread (7 x 300 x 800 over axis 1: 8.4 us against 48); with more
-    // outputs, and for other patterns, a thread per output keeps memory busy by itself.
+    // workgroup that still give every CU one), from 16 elements on, or 8 in 16-byte loads (30,000 rows
+    // of 9 take 5.2 us so and 3.9 with a thread each).  Columns do where a thread per output, which
+    // batches 16 loads, is short of them: up to 64 elements (16 x 40 x 130 over axis 1: 3.3 us
+    // against 4.0; 16 x 200 x 130 8.4 against 6.9) or with so few columns in many places that its
+    // loads hardly coalesce (300 x 200 x 2: 8.6 against 24; 16 of them 8.4 against 7.0), and not past 1,024 workgroups (30,000 x 40 x 2, two
+    // lanes of a workgroup each: 30 us against 7.3).
     const float* x = (const float*)l.in0;
     float* y = (float*)l.out;
-    if (p.rr == 1 && p.rk <= 1 && inner == 1 && p.rcount >= 8) {
+    const bool row_vec = p.rcount % 4 == 0 && ((uintptr_t)x & 15) == 0;
+    if (p.rr == 1 && p.rk <= 1 && inner == 1 && p.rcount >= (row_vec ? 8 : 16)) {
         int rows = 256;
         while (rows > 4 && (outer + rows - 1) / rows < 256) rows /= 2;
         while (rows > 4 && rows * p.rcount >= (1ll << 28)) rows /= 2;  // 32-bit offsets
         const int64_t wgs = (outer + rows - 1) / rows;
         if (wgs < (1ll << 31) && rows * p.rcount < (1ll << 28)) {
             const int n = (int)p.rcount;
-            const bool vec = n % 4 == 0 && ((uintptr_t)x & 15) == 0;
-            auto kern = p.kind ? (vec ? reduce_rows_kernel<true, true> : reduce_rows_kernel<false, true>)
-                               : (vec ? reduce_rows_kernel<true, false> : reduce_rows_kernel<false, false>);
+            auto kern = p.kind ? (row_vec ? reduce_rows_kernel<true, true> : reduce_rows_kernel<false, true>)
+                               : (row_vec ? reduce_rows_kernel<true, false> : reduce_rows_kernel<false, false>);
             hipLaunchKernelGGL(kern, dim3((unsigned)wgs), dim3(256), 0, l.stream, x, y, p.init, outer,
                                n, rows);
             SHP_HIP_CHECK(hipGetLastError());
             return SHP_OK;
         }
     }
-    if (p.rr == 1 && inner > 1 && inner < (1 << 30) && p.rcount >= 16 && kept <= 65536) {
+    const int64_t col_wgs = outer * ((inner + 63) / 64);
+    if (p.rr == 1 && inner > 1 && p.rcount > 16 && col_wgs <= 1024 &&
+        (p.rcount < 64 || (inner <= 3 && outer >= 64))) {
         const int blocks = (int)((inner + 63) / 64);
         hipLaunchKernelGGL(reduce_cols_kernel, dim3((unsigned)(outer * blocks)), dim3(256), 0,
                            l.stream, x, y, p.kind, p.init, (int)p.rcount, (int)inner, blocks);

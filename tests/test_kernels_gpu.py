@@ -989,7 +989,12 @@ def test_hlo_select(ctx, orc):
                                         # columns through LDS tiles and by thread, merged axes
                                         ((2, 65, 130), (1,)), ((7, 27, 138), (0, 1)), ((1, 64, 1, 63), (1,)),
                                         ((2, 16, 40000), (1,)), ((4, 130, 3, 1, 5), (1,)),
-                                        ((2, 40, 3, 50), (1, 3)), ((6, 1, 4), (1,))])
+                                        ((2, 40, 3, 50), (1, 3)), ((6, 1, 4), (1,)),
+                                        # on both sides of the lines between those forms
+                                        ((2, 63, 130), (1,)), ((2, 64, 130), (1,)), ((5, 17, 64), (1,)),
+                                        ((5, 16, 64), (1,)), ((1024, 40, 2), (1,)), ((1025, 40, 2), (1,)),
+                                        ((300, 200, 3), (1,)), ((300, 200, 4), (1,)), ((63, 200, 2), (1,)),
+                                        ((70, 15), (1,)), ((70, 12), (1,)), ((70, 17), (1,))])
 def test_hlo_reduce(ctx, orc, shape, dims):
     """Sum folds in source order on both sides, so it is bit-exact like max."""
     from spirv_inference_amd import hlo_ops as H
