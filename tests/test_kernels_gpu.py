@@ -1036,6 +1036,16 @@ def test_row_kernels_all_widths(ctx, orc, rows, cols):
         assert_close(y, r, 1e-4, 1e-4, f"{k} {rows}x{cols}")
 
 
+@pytest.mark.parametrize("rows,cols", [(2047, 513), (2048, 513), (2048, 1001), (1, 512), (2050, 511)])
+def test_row_norms_of_many_unaligned_rows(ctx, orc, rows, cols):
+    """A wavefront or a workgroup per row, by the number of rows."""
+    x, w = rnd(rows, cols) * 2, rnd(2 * cols)
+    eb = int(np.array([1e-12], np.float32).view(np.int32)[0])
+    for k, b in (("layernorm_rows", w), ("rmsnorm_rows", w[:cols])):
+        y, r = both(ctx, orc, k, x, b, rows * cols, [rows, cols, eb])
+        assert_close(y, r, 1e-4, 1e-4, f"{k} {rows}x{cols}")
+
+
 GATHERS = [((3, 5, 7, 64), (0, 2, 1, 3)), ((3, 5, 7, 33), (0, 2, 1, 3)), ((2, 70, 12, 64), (0, 2, 3, 1)),
            ((2, 70, 12, 33), (0, 3, 2, 1)), ((1, 300, 4, 64), (0, 1, 3, 2)), ((7, 9, 130, 3), (2, 0, 1, 3)),
            ((65, 129), (1, 0)), ((300, 5), (1, 0)), ((5, 300), (1, 0)), ((2, 3, 2, 5, 3, 4), (5, 0, 3, 1, 4, 2)),
