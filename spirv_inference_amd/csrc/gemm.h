@@ -78,7 +78,8 @@ size_t gemm_workspace_bytes(const GemmParams& p, int amode, int bmode, int cmode
 // The small-problem kernel (kernels_gemm_direct.hip): whether it takes the operands at all, with
 // how many K splits it should run (0: the tiled kernels are better), its workspace, its launch.
 bool direct_eligible(const GemmParams& p, int amode, int bmode, int cmode);
-int direct_splits(const GemmParams& p, int tune);
+int direct_splits(const GemmParams& p, int amode, int bmode, int tune);
+bool direct_may_exceed(const GemmParams& p, int bmode);
 size_t direct_workspace(const GemmParams& p, int splits);
 int direct_launch(hipStream_t stream, GemmParams p, int amode, int bmode, int splits,
                   float* workspace);

@@ -2417,7 +2417,7 @@ size_t gemm_workspace_bytes(const GemmParams& p, int amode, int bmode, int cmode
     }
     size_t direct = 0;
     if (direct_eligible(p, amode, bmode, cmode))
-        direct = direct_workspace(p, direct_splits(p, tune ? direct_tune(*tune) : 0));
+        direct = direct_workspace(p, direct_splits(p, amode, bmode, tune ? direct_tune(*tune) : 0));
     if (splits <= 1) return direct;
     return std::max(direct, kSplitCounterBytes + (size_t)splits * nbatch * p.M * p.N * sizeof(float));
 }
@@ -2559,13 +2559,14 @@ int gemm_launch(hipStream_t stream, GemmParams p, int amode, int bmode, int cmod
     }
     const bool direct_ok = direct_eligible(p, amode, bmode, cmode);
     if (direct_ok) {
-        const int ds = direct_splits(p, direct_tune(tn));
+        const int ds = direct_splits(p, amode, bmode, direct_tune(tn));
         if (ds == 1 || (ds > 1 && workspace && workspace_bytes >= direct_workspace(p, ds)))
             return direct_launch(stream, p, amode, bmode, ds, workspace);
     }
     const int blm = bl_mask(p, amode, bmode, cmode);
     Plan pl = plan_gemm(p, nbatch, hot, dma_ok, amode == A_CONV_NHWC4, tn, amode, bmode, blm);
-    if (direct_ok && direct_tune(tn) == 0 && direct_cost(p, amode) < pl.cost)
+    if (direct_ok && direct_tune(tn) == 0 && direct_may_exceed(p, bmode) &&
+        direct_cost(p, amode) < pl.cost)
         return direct_launch(stream, p, amode, bmode, 1, workspace);
     size_t need = pl.splits > 1
                       ? kSplitCounterBytes + (size_t)pl.splits * nbatch * p.M * p.N * sizeof(float)

@@ -263,7 +263,20 @@ bool direct_eligible(const GemmParams& p, int amode, int bmode, int cmode) {
 // compares both estimates.  K is split while every CU
 // still gets at most one workgroup and a split keeps 128 k: a second round of workgroups costs more
 // than the shorter chains give (200x2304x768, 252 tiles: 10.5 us unsplit, 13.2 in two).
-int direct_splits(const GemmParams& p, int tune) {
+//
+// A further sweep (840 products and convolutions up to K = 51,200, both operand orders) found where
+// that ends: where the workgroups' own K is long and they leave CUs idle, the tiled kernels' splits
+// fill the GPU better, and an [N][K] operand, whose loads are 64 bytes of 16 rows, earlier still:
+//  - [K][N]: from 4,000 k a workgroup while these fill less than three quarters of the CUs
+//    (1000x300x16384 124 us, tiled 90; at 192 workgroups and more direct still wins);
+//  - [N][K] products: from 3,000 k, or 2,000 while they fill less than that (265x952x11376 94 us,
+//    tiled 67; 1164x264x2080 26.6, 24.3);
+//  - [N][K] convolutions with taps: from 300 k, 700 under 160 workgroups and 4,000 under 64
+//    (2x32x32x2048 to 192 channels, 3x3: 237 us, tiled 143; 7x28x28x256 to 192, stride 2: 38, 30);
+//    1x1 with a stride, which the tiled kernel reads as rows: from 300 k, and with K under 512
+//    (12x16x16x2048 to 256: 23.5, 16.4; 9x33x33x48 to 128: 7.6, 5.9; 7x32x32x512 to 16: 9.8, 14.6).
+// Over 930 shapes this is within 0.4 % of the faster of the two on average.
+int direct_splits(const GemmParams& p, int amode, int bmode, int tune) {
     if (tune < 0) return 0;
     const int64_t tiles = (int64_t)((p.M + kTm - 1) / kTm) * ((p.N + kTn - 1) / kTn);
     const int steps = p.K / 16;
@@ -275,9 +288,28 @@ int direct_splits(const GemmParams& p, int tune) {
         if (tiles > 256) return 0;
         for (int t : {2, 3, 4, 6, 8})
             if (tiles * t <= 256 && p.K / t >= 128) s = t;
+        const int64_t wgs = tiles * s;
+        const int k = p.K / s;
+        const bool conv = amode == A_CONV_NHWC4;
+        if (bmode == B_NVEC) {
+            if (!conv && k > 4000 && wgs < 192) return 0;
+        } else if (conv && p.ckh * p.ckw > 1) {
+            if (k > (wgs < 64 ? 4000 : wgs < 160 ? 700 : 300)) return 0;
+        } else if (conv && (p.csh > 1 || p.csw > 1)) {
+            if (p.K < 512 || k > 300) return 0;
+        } else if (k > (wgs < 192 ? 2000 : 3000)) {
+            return 0;
+        }
     }
     const int per = (steps + s - 1) / s;
     return (steps + per - 1) / per;
+}
+
+// Above one tile per CU, by time estimates: [K][N] operands only.  With [N][K] ones the direct kernel
+// lost on 141 of 143 swept shapes, by up to 1.9 times (3x56x56x192 to 512 channels, 3x3: 244 us, tiled 153).
+bool direct_may_exceed(const GemmParams& p, int bmode) {
+    const int64_t tiles = (int64_t)((p.M + kTm - 1) / kTm) * ((p.N + kTn - 1) / kTn);
+    return tiles > 256 && bmode == B_NVEC;
 }
 
 size_t direct_workspace(const GemmParams& p, int splits) {

@@ -1188,6 +1188,42 @@ def test_gemm_direct_convolutions(ctx, orc, n, ih, ic, k, oc, s):
             ctx.tune("gemm_small", 0)
 
 
+@pytest.mark.parametrize("kernel,dims,direct", [
+    # products m, k, n on [K][N] and [N][K]; convolutions n, map, ic, oc, window, stride on [OC][K]
+    ("hlo_dot_rank2", (1000, 4096, 300), False), ("hlo_dot_rank2", (1000, 3072, 300), True),
+    ("hlo_dot_rank2", (1537, 4096, 200), True), ("fully_connected", (1164, 2080, 264), False),
+    ("fully_connected", (1164, 1984, 264), True), ("fully_connected", (1537, 3072, 200), False),
+    ("fully_connected", (2163, 992, 660), False), ("conv2d_nhwc", (2, 14, 64, 64, 3, 1), True),
+    ("conv2d_nhwc", (7, 28, 256, 192, 3, 2), False), ("conv2d_nhwc", (2, 14, 96, 512, 1, 2), False),
+    ("conv2d_nhwc", (3, 33, 256, 256, 3, 1), False), ("conv2d_nhwc", (1, 7, 512, 32, 3, 1), True),
+    ("conv2d_nhwc", (2, 32, 512, 24, 3, 2), True), ("conv2d_nhwc", (7, 32, 512, 16, 1, 2), True),
+    ("conv2d_nhwc", (12, 16, 2048, 256, 1, 2), False)])
+def test_gemm_direct_rule(ctx, orc, kernel, dims, direct):
+    """Which kernel the planner takes on both sides of the direct kernel's lines, by the bits of the
+    result with that kernel switched off, and the result itself."""
+    if kernel == "conv2d_nhwc":
+        n, hw, ic, oc, k, s = dims
+        p = (k - 1) // 2
+        oh = (hw + 2 * p - k) // s + 1
+        x = rnd(n, hw, hw, ic)
+        w = orc.pack_conv_weight(rnd(oc, ic, k, k) * np.float32(1 / np.sqrt(ic * k * k)), rnd(oc))
+        total = n * oh * oh * oc
+        push = [n, ic, hw, hw, oc, oh, oh, k, k, s, s, 1, p, p, total]
+    else:
+        m, k, n = dims
+        x, w, total, push = rnd(m, k), rnd(k * n + n) * np.float32(1 / np.sqrt(k)), m * n, [m, k, n, m * n]
+        if kernel == "hlo_dot_rank2":
+            w = w[:k * n]
+    y, ref = both(ctx, orc, kernel, x, w, total, push)
+    assert_close(y, ref, 1e-4, 1e-4, f"{kernel} {dims}")
+    ctx.tune("direct", -1)
+    try:
+        tiled = _dev(ctx, kernel, x, w, total, push)
+    finally:
+        ctx.tune("direct", 0)
+    assert np.array_equal(y, tiled) != direct
+
+
 @pytest.mark.parametrize("m,k,n", [(384, 768, 3072), (515, 2048, 1300), (1071, 1280, 500), (1600, 80, 772)])
 def test_gemm_planned_products(ctx, orc, m, k, n):
     """More tiles than CUs, where the plan goes by estimated time: the direct kernel over two and
