@@ -740,32 +740,45 @@ const TunedBlock* tuned_block(const IrShape& sh) {
 }
 
 // Whether one launch is expected to beat the separate ones: the measured verdict for the blocks
-// above; elsewhere rules on sizes, fitted to the 21 distinct blocks of MobileNetV2 and
-// EfficientNet-Lite0 at batches 1-32, each as one launch, as expand GEMM + depthwise/projection
-// launch and as three launches (graph-replayed; the rules' sums lie within 4 % of the fastest form
-// per block at every batch).  A whole block pays
-// * with cin <= 24 at any size: the expand is thin and memory bound, its output six times the input;
-// * with cin <= 48 up to 2,000 input pixels (1x28x28x32: 10.0 us against 12.8 in three launches;
-//   4x28x28x32 to 64: 17.5 against 13.7);
-// * beyond, where the launches are latencies: 3x3, ce under 900, cin * pixels up to 37,000
-//   (1x14x14x96: 14.0 against 14.7; 4x14x14x96: 22.1 against 18.8; 12x7x7x192: 63.2 against 27.9).
-// The depthwise + projection form (no expand) pays with ce <= 96 on maps of 56x56 and more, the
-// only ones measured; at stride 1 up to ce 256 (24x56x56x144: 0.87 of the two launches) and up to
-// ce 700 while the projection is small (4x14x14x384: 0.95, 12x14x14x384: 1.15); at stride 2 up to
-// ce 256 for few outputs, more of them with a 5x5 window, whose taps the fused form reads from LDS.
+// above; elsewhere rules on sizes, fitted to 1,750 blocks (the distinct ones of MobileNetV2 and
+// EfficientNet-Lite0 and MobileNetV1's pairs at batches 1-32, and 1,510 of other maps, widths and
+// batches), each as one launch, as expand GEMM + depthwise/projection launch and as three launches
+// (graph-replayed).  The form chosen lies within 2 % of the fastest on average; a rule fitted to the
+// two networks alone lay at 10 % and lost up to 4.7 times, on wide outputs: the fused form's projection
+// runs on a few pixels at a time, so its products (`proj`, multiply-adds) must be few or narrow.
+// A whole block pays
+// * with cin <= 24, whose expand is thin and memory bound, its output several times the input;
+// * with cin <= 48 on large maps to few channels (32x28x28x32: 30.1 us, 42.2 in three launches) and
+//   on small inputs;
+// * beyond, where the launches are latencies (3x14x14x64: 13.7 us, 15.8).
+// The depthwise + projection form (no expand) pays to few channels once there is work to fuse, and where
+// the whole is small (4x14x14x384 to 64: 0.9 of two launches); 4x75x75x80 to 320 takes 120 us so, 33
+// in two.  With a 5x5 window, whose taps the fused form reads from LDS, further up.
 bool fusion_pays(const IrShape& sh) {
     if (const TunedBlock* t = tuned_block(sh)) return t->fuse;
     const int64_t in = (int64_t)sh.n * sh.h * sh.w, out = (int64_t)sh.n * sh.oh * sh.ow;
+    const int64_t mid = out * sh.ce, proj = mid * sh.cout;
+    const bool down = sh.s > 1;
     if (sh.expand) {
-        if (sh.cin <= 24) return true;
-        if (sh.cin <= 48) return in <= 2000;
-        return sh.k == 3 && sh.ce < 900 && sh.cin * in <= 37000;
+        if (sh.cin <= 24) {
+            if (proj <= 8000000) return true;
+            if (sh.k == 5 && !down) return sh.cout <= 72 && sh.ce <= 112;
+            return sh.cout <= (down ? 160 : 72);
+        }
+        if (sh.cin <= 48)
+            return (in > 10000 && sh.cout <= (down ? 128 : 48)) ||
+                   (in <= 2000 && sh.cout <= 96 && (sh.k == 3 || proj <= 20000000));
+        return sh.k == 3 && sh.ce < 900 && sh.cin * in <= 37000 && proj <= 12000000;
     }
-    if (sh.ce <= 96) return out >= 3000;
-    if (sh.s == 1)
-        return sh.ce <= 256 || (sh.ce <= 480 && out <= (sh.k == 5 ? 1600 : 1200)) ||
-               (sh.ce <= 700 && out <= 800);
-    return sh.ce <= 256 && out <= (sh.k == 5 ? 6300 : 400);
+    if (sh.k == 3)
+        return down ? sh.cout <= 52 && out > 4500
+                    : (sh.cout <= 56 && mid > 320000) ||
+                          (sh.ce > 216 && sh.ce <= 700 && proj <= 25000000);
+    if (!down)
+        return (proj <= 60000000 && sh.ce * sh.cout <= 150000 &&
+                sh.cout <= std::min(256, 4 * sh.ce)) ||
+               (sh.cout <= 44 && mid > 6000000);
+    return proj <= 13000000 || (proj <= 60000000 && sh.cout <= 144 && out <= 7400);
 }
 
 IrPlan choose_plan(const IrShape& sh, const shp::GemmTune& tn, bool allow_split) {

@@ -72,3 +72,29 @@ def test_product_does_not_link_the_oracle():
     assert b"liboracle" not in blob and b"orc_run_kernel" not in blob
     src = "\n".join(p.read_text() for p in (ROOT / "spirv_inference_amd").rglob("*.py"))
     assert "import oracle" not in src and "from oracle" not in src
+
+
+@pytest.mark.parametrize("n,hw,cin,ce,cout,k,s,whole,pair", [
+    # measured on the GPU, graph-replayed: three launches / expand + one / one launch, us
+    (4, 75, 80, 80, 320, 3, 1, None, False),    # 33 / 120
+    (8, 112, 128, 128, 192, 3, 1, None, False),  # 93 / 162
+    (21, 112, 64, 64, 192, 3, 2, None, False),  # 48 / 93
+    (16, 14, 96, 96, 96, 3, 1, None, False),    # a batch of small maps is no large map
+    (14, 112, 40, 160, 320, 3, 1, False, False),  # 309 / 908 / 743
+    (32, 28, 32, 192, 32, 3, 1, True, True),    # 42 / 36 / 30
+    (1, 56, 24, 144, 32, 3, 1, True, True),
+    (13, 14, 16, 16, 512, 5, 1, None, False),
+    (5, 14, 512, 512, 48, 5, 1, None, True)])
+def test_block_verdicts(n, hw, cin, ce, cout, k, s, whole, pair):
+    """Which form of an MBConv block shp_block_plan expects to be faster, outside the measured tables:
+    the whole block, and its depthwise + projection pair, against separate launches."""
+    from spirv_inference_amd import lib
+    oh = (hw + s - 1) // s
+    pad = max((oh - 1) * s + k - hw, 0) // 2
+    out = (C.c_int32 * 8)()
+    for expand, inp, want in ((1, cin, whole), (0, ce, pair)):
+        if want is None:
+            continue
+        push = [n, inp, hw, hw, ce, cout, oh, oh, k, s, pad, pad, expand, 2, 2, n * oh * oh * cout]
+        assert lib().shp_block_plan((C.c_int32 * 16)(*push), 16, out) == 0
+        assert bool(out[7]) == want, push
