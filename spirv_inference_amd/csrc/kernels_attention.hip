@@ -113,7 +113,9 @@ __global__ __launch_bounds__(U * 128) void attention_kernel(AttnArgs a, int wgs,
         for (int i = 0; i < NST; ++i) {
             const int e = i * T + tid, row = e >> 4, d = (e & 15) * 4;
             *reinterpret_cast<f4v*>(&Ks[row * kRs + d]) = ks[i];
-            *reinterpret_cast<f4v*>(&Vs[row * kRs + d]) = vs[i];
+            // past the last key the weight is 0, which must not meet the last row's infinity
+            *reinterpret_cast<f4v*>(&Vs[row * kRs + d]) =
+                t * 2 * kKeys + row < a.n_keys ? vs[i] : f4v{0.f, 0.f, 0.f, 0.f};
         }
         if constexpr (MASK)
             if (tid < 2 * kKeys) Ms[tid] = ms;

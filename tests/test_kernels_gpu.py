@@ -657,6 +657,21 @@ def test_attention_rows(ctx, orc, S, masked):
     assert_close(y[cols], r[cols], 1e-4, 1e-4, f"attention_rows S={S} {masked}")
 
 
+@pytest.mark.parametrize("S", [5, 64, 65, 128, 130, 200])
+def test_attention_rows_infinite_last_value(ctx, orc, S):
+    """An infinity in the last key's V stays an infinity in its column, and touches no other."""
+    B, H, HD = 1, 2, 64
+    qkv = rnd(B, S, 3, H, HD)
+    qkv[0, S - 1, 2, 1, 7] = np.inf
+    ld = 3 * H * HD
+    push = [B, H, S, HD, ld, 0, H * HD, 2 * H * HD, H * HD, int(np.float32(0.125).view(np.int32)), B * S * H * HD]
+    y = _dev(ctx, "attention_rows", qkv, None, push[10], push).reshape(S, H * HD)
+    want = orc.run("attention_rows", qkv, None, push[10], push).reshape(S, H * HD)
+    assert (y[:, HD + 7] == np.inf).all() and (want[:, HD + 7] == np.inf).all()
+    keep = np.arange(H * HD) != HD + 7
+    assert_close(y[:, keep], want[:, keep], 1e-4, 1e-4, f"S {S}")
+
+
 def test_attention_fused_rejects_other_sequence_lengths(ctx):
     from spirv_inference_amd import ShpError
     S, HD, B, H = 64, 64, 1, 2
