@@ -313,9 +313,9 @@ def test_llama_small_tokens_and_logits(ctx, orc, engine):
         assert lm.generate(prompt, 8) == (want[:stop[0]] if stop else want)
 
 
-@pytest.mark.parametrize("n", [2, 15, 16, 17, 33, 64, 65, 130, 512, 513, 600])
+@pytest.mark.parametrize("n", [3, 15, 16, 17, 33, 64, 65, 130, 512, 513, 600])
 def test_llama_prompt_pass_equals_token_steps(ctx, n):
-    """generate() takes the whole prompt in one pass (up to 64 rows per product on the
+    """generate() takes a prompt of three ids and more in one pass (up to 64 rows per product on the
     weight-streaming kernel, above on the tiled ones, 512 positions per chunk); the argmax of every
     position, the KV cache and the last logits equal those of the prompt fed one step per id."""
     from spirv_inference_amd.models import Llama
@@ -344,6 +344,48 @@ def test_llama_prompt_pass_equals_token_steps(ctx, n):
         got = state()
         for k, w in want.items():
             assert_close(got[k].ravel(), w.ravel(), 1e-4, 1e-4, f"prompt of {n}: {k}")
+        # it was the pass: token steps of the default engine give up at this limit
+        assert lm.engine == "persistent"
+        lm.set_wait_limit(0)
+        lm.generate(prompt, 1)
+        assert lm.tokens() == tokens[:n]
+        lm.set_wait_limit(-1)
+
+
+def test_llama_prompt_of_two_ids_takes_token_steps(ctx):
+    """Two steps are shorter than a pass: the same logits bit for bit."""
+    from spirv_inference_amd.models import Llama
+    with Llama(ctx, seed=9, **SMALL) as lm:
+        lm.reset()
+        for t in (17, 401):
+            lm.step(t)
+        ctx.sync()
+        tokens, want = lm.tokens(), lm.logits()
+        lm.generate([17, 401], 1)
+        assert lm.tokens() == tokens
+        np.testing.assert_array_equal(lm.logits(), want)
+
+
+@pytest.mark.parametrize("n,heads", [(368, 32), (369, 32), (401, 32), (420, 28)])
+def test_llama_prompt_pass_of_many_heads(ctx, n, heads):
+    """32 query heads on 4 KV heads: from 369 ids on four units of 16 queries share a workgroup's keys
+    in the causal attention.  With 28 heads and 420 ids the last workgroup has one unit."""
+    from spirv_inference_amd.models import Llama
+    cfg = dict(SMALL, hidden=64, n_heads=heads, n_kv_heads=4, ffn=64, vocab=304, max_seq=512)
+    prompt = [int(t) for t in np.random.default_rng(n).integers(3, cfg["vocab"], n)]
+    with Llama(ctx, seed=9, **cfg) as lm:
+        lm.reset()
+        for t in prompt:
+            lm.step(t)
+        ctx.sync()
+        tokens, want = lm.tokens(), lm.logits()
+        kv = [lm.weight(1, w).reshape(4, -1)[:, :n * 64] for w in ("k_cache", "v_cache")]
+        lm.generate(prompt, 1)
+        assert lm.tokens() == tokens
+        assert_close(lm.logits(), want, 1e-4, 1e-4, f"prompt of {n}")
+        for w, c in zip(("k_cache", "v_cache"), kv):  # layer 1 reads layer 0's attention at every position
+            got = lm.weight(1, w).reshape(4, -1)[:, :n * 64]
+            assert_close(got.ravel(), c.ravel(), 1e-4, 1e-4, f"prompt of {n}: {w}")
 
 
 @pytest.mark.parametrize("hidden,ffn,vocab", [(8, 4, 8), (16, 12, 24), (72, 20, 40)])
