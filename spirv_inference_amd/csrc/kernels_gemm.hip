@@ -2228,19 +2228,17 @@ double direct_cost(const GemmParams& p, int amode) {
 }
 
 // Plans measured best on MI355X for the benchmark configs' shapes: sweeps of every tile, K
-// tile and split count of both kernels per shape, with split counts down to one K tile per
-// split for the 1x1 convolutions of MobileNetV2 b1 and EfficientNet-Lite0 b8.  An entry only
-// where the best plan beat the cost model's by more than 2.5 % alone and did not lose inside
-// the model's forward pass; the cost model decides every other shape.  Key: operand modes,
-// batch count, M, N, K, and for convolutions the input channels, stride and kernel height (0
-// for products).
+// tile and split count of both kernels per shape.  An entry only where the best plan beat the
+// cost model's by more than 2.5 % alone and did not lose inside the model's forward pass; the
+// cost model decides every other shape.  The networks' stems and small 1x1 convolutions never come
+// here: their own kernels take them.  Key: operand modes, batch count, M, N, K, and for
+// convolutions the input channels, stride and kernel height (0 for products).
 struct TunedPlan {
     int amode, bmode, nbatch, M, N, K, cic, csh, ckh;
     TileCfg t;
     int splits;
 };
 const TunedPlan kTuned[] = {
-{shp::A_CONV_NHWC, shp::B_NVEC, 1, 401408, 64, 147, 3, 2, 7, {64, 64, 32, false, 1, false}, 1},  // resnet50_v1_5 conv1: 146.1 vs 156.1 us
     {shp::A_CONV_NHWC4, shp::B_NVEC, 1, 100352, 64, 576, 64, 1, 3, {64, 64, 16, false, 1, true}, 1},  // resnet50_v1_5 conv2_block1_2: 80.4 vs 87.6 us
     {shp::A_CONV_NHWC4, shp::B_NVEC, 1, 25088, 128, 1152, 128, 2, 3, {64, 64, 16, false, 1, true}, 2},  // resnet50_v1_5 conv3_block1_2: 83.2 vs 89.6 us
     {shp::A_CONV_NHWC4, shp::B_NVEC, 1, 25088, 128, 1152, 128, 1, 3, {64, 64, 16, false, 1, true}, 3},  // resnet50_v1_5 conv3_block2_2: 82.5 vs 93.4 us
@@ -2251,44 +2249,19 @@ const TunedPlan kTuned[] = {
     {shp::A_CONV_NHWC4, shp::B_NVEC, 1, 1568, 2048, 1024, 1024, 2, 1, {64, 64, 32, false, 1, true}, 1},  // resnet50_v1_5 conv5_block1_0: 69.2 vs 71.2 us
     {shp::A_KVEC, shp::B_KVEC, 96, 128, 128, 64, 0, 0, 0, {64, 64, 16, false, 1, true}, 1},  // bert_base layer0_scores: 9.4 vs 9.9 us
     {shp::A_KVEC, shp::B_NVEC, 96, 128, 64, 128, 0, 0, 0, {64, 64, 16, false, 1, true}, 1},  // bert_base layer0_context: 8.7 vs 9.1 us
-    {shp::A_CONV_NHWC, shp::B_STRIDED, 1, 100352, 32, 27, 3, 2, 3, {64, 64, 32, false, 1, false}, 1},  // efficientnet_lite0 stem: 21.4 vs 22.2 us
     {shp::A_CONV_NHWC4, shp::B_KVEC, 1, 100352, 96, 16, 16, 1, 1, {64, 64, 16, false, 1, true}, 1},  // efficientnet_lite0 block1_expand: 19.2 vs 19.7 us
-    {shp::A_CONV_NHWC4, shp::B_KVEC, 1, 6272, 240, 40, 40, 1, 1, {64, 64, 16, false, 1, false}, 1},  // efficientnet_lite0 block4_expand: 10.6 vs 11.5 us
-    {shp::A_CONV_NHWC4, shp::B_KVEC, 1, 1568, 80, 480, 480, 1, 1, {64, 64, 16, false, 1, true}, 5},  // efficientnet_lite0 block6_project: 12.2 vs 15.3 us
-    {shp::A_CONV_NHWC4, shp::B_KVEC, 1, 1568, 112, 480, 480, 1, 1, {64, 64, 16, false, 1, true}, 5},  // efficientnet_lite0 block8_project: 12.8 vs 15.0 us
-    {shp::A_CONV_NHWC4, shp::B_KVEC, 1, 1568, 672, 112, 112, 1, 1, {64, 64, 16, false, 1, true}, 1},  // efficientnet_lite0 block9_expand: 11.2 vs 11.5 us
-    {shp::A_CONV_NHWC4, shp::B_KVEC, 1, 392, 1152, 192, 192, 1, 1, {64, 64, 32, false, 1, true}, 1},  // efficientnet_lite0 block12_expand: 10.5 vs 11.1 us
-    {shp::A_CONV_NHWC4, shp::B_KVEC, 1, 392, 192, 1152, 1152, 1, 1, {64, 64, 16, false, 1, true}, 6},  // efficientnet_lite0 block12_project: 13.6 vs 13.9 us
-    {shp::A_CONV_NHWC4, shp::B_KVEC, 1, 392, 320, 1152, 1152, 1, 1, {64, 64, 16, false, 1, true}, 6},  // efficientnet_lite0 block15_project: 14.2 vs 14.8 us
-    {shp::A_CONV_NHWC4, shp::B_KVEC, 1, 392, 1280, 320, 320, 1, 1, {64, 64, 32, false, 1, true}, 1},  // efficientnet_lite0 head_conv: 12.9 vs 13.3 us
-    {shp::A_CONV_NHWC, shp::B_STRIDED, 1, 12544, 32, 27, 3, 2, 3, {64, 64, 32, false, 1, false}, 1},  // mobilenet_v2 stem: 8.6 vs 8.8 us
-    {shp::A_CONV_NHWC4, shp::B_KVEC, 1, 12544, 16, 32, 32, 1, 1, {64, 64, 16, false, 1, true}, 1},  // mobilenet_v2 block0_project: 7.3 vs 7.5 us
-    {shp::A_CONV_NHWC4, shp::B_KVEC, 1, 3136, 24, 96, 96, 1, 1, {64, 64, 16, false, 1, true}, 1},  // mobilenet_v2 block1_project: 8.4 vs 8.7 us
-    {shp::A_CONV_NHWC4, shp::B_KVEC, 1, 196, 64, 192, 192, 1, 1, {64, 64, 16, false, 1, true}, 1},  // mobilenet_v2 block6_project: 10.0 vs 10.7 us
-    {shp::A_CONV_NHWC4, shp::B_KVEC, 1, 196, 384, 64, 64, 1, 1, {64, 64, 16, false, 1, true}, 1},  // mobilenet_v2 block7_expand: 7.8 vs 8.4 us
-    {shp::A_CONV_NHWC4, shp::B_KVEC, 1, 196, 64, 384, 384, 1, 1, {64, 64, 32, false, 1, true}, 6},  // mobilenet_v2 block7_project: 11.0 vs 13.6 us
-    {shp::A_CONV_NHWC4, shp::B_KVEC, 1, 196, 96, 384, 384, 1, 1, {64, 64, 16, false, 1, true}, 6},  // mobilenet_v2 block10_project: 10.6 vs 13.4 us
-    {shp::A_CONV_NHWC4, shp::B_KVEC, 1, 196, 576, 96, 96, 1, 1, {64, 64, 16, false, 1, true}, 1},  // mobilenet_v2 block11_expand: 8.5 vs 9.0 us
-    {shp::A_CONV_NHWC4, shp::B_KVEC, 1, 196, 96, 576, 576, 1, 1, {64, 64, 32, false, 1, true}, 5},  // mobilenet_v2 block11_project: 11.7 vs 12.3 us
-    {shp::A_CONV_NHWC4, shp::B_KVEC, 1, 49, 160, 576, 576, 1, 1, {64, 64, 16, false, 1, true}, 5},  // mobilenet_v2 block13_project: 11.7 vs 12.2 us
-    {shp::A_CONV_NHWC4, shp::B_KVEC, 1, 49, 960, 160, 160, 1, 1, {64, 64, 16, false, 1, true}, 1},  // mobilenet_v2 block14_expand: 9.5 vs 9.9 us
-    {shp::A_CONV_NHWC4, shp::B_KVEC, 1, 49, 160, 960, 960, 1, 1, {64, 64, 16, false, 1, true}, 8},  // mobilenet_v2 block14_project: 12.4 vs 14.1 us
-    {shp::A_CONV_NHWC4, shp::B_KVEC, 1, 49, 320, 960, 960, 1, 1, {64, 64, 16, false, 1, true}, 6},  // mobilenet_v2 block16_project: 12.4 vs 13.0 us
-    {shp::A_CONV_NHWC4, shp::B_KVEC, 1, 49, 1280, 320, 320, 1, 1, {64, 64, 16, false, 1, true}, 5},  // mobilenet_v2 head_conv: 10.8 vs 12.3 us
 };
 
 // The table's plan for this problem, if it has one that the problem's operands allow.
-bool tuned_plan(const GemmParams& p, int nbatch, int amode, int bmode, bool hot, int blm,
-                Plan* out) {
+bool tuned_plan(const GemmParams& p, int nbatch, int amode, int bmode, int blm, Plan* out) {
     for (const TunedPlan& e : kTuned) {
         if (e.amode != amode || e.bmode != bmode || e.nbatch != nbatch || e.M != p.M ||
             e.N != p.N || e.K != p.K)
             continue;
         if (e.cic && (e.cic != p.cic || e.csh != p.csh || e.ckh != p.ckh)) continue;
         const TileCfg& t = e.t;
-        if (t.bl && !(blm & (t.bk == 16 ? 1 : t.bk == 32 ? 2 : 4))) return false;
-        if (!t.bl && !hot && (t.bk != 32 || t.pg > 1)) return false;
-        const int kq = t.bl && t.bk == 64 ? 64 : 32;
+        if (!(blm & (t.bk == 16 ? 1 : t.bk == 32 ? 2 : 4))) return false;
+        const int kq = t.bk == 64 ? 64 : 32;
         int kps = ((p.K + e.splits - 1) / e.splits + kq - 1) / kq * kq;
         if ((p.K + kps - 1) / kps != e.splits) return false;
         *out = Plan{t, e.splits, kps, 0};
@@ -2350,7 +2323,7 @@ Plan plan_gemm(const GemmParams& p, int nbatch, bool hot, bool dma_ok, bool conv
     static const int kTiles[5][2] = {{128, 128}, {128, 64}, {64, 64}, {128, 128}, {128, 64}};
     Plan tuned;
     if (tn.table >= 0 && !tn.tile && !tn.bk && !tn.splits && !tn.dma && !tn.pg && !tn.bl &&
-        tuned_plan(p, nbatch, amode, bmode, hot, blm, &tuned))
+        tuned_plan(p, nbatch, amode, bmode, blm, &tuned))
         return tuned;
     if (blm && tn.bl >= 0 && (tn.bl > 0 || (tn.dma <= 0 && !tn.pg)) &&
         plan_bl(p, nbatch, amode, blm, tn, &tuned))
