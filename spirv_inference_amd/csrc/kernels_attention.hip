@@ -15,7 +15,7 @@
 //
 // Measured (MI355X, graph-replayed): 96 heads x 128 queries 14.1 -> 10.6 us against a kernel that
 // staged a whole head's K and V and sent P through LDS, 36 x 200 27 (three operators) -> 11.7 us; a
-// causal prompt of 384 (32 heads on 4 KV heads) 33 -> 12 us with the keys halved over a pair.
+// causal prompt of 384 (32 heads on 4 KV heads) 23 us in the kernel trace.
 //
 // The arithmetic is the three-operator chain's apart from the order of the sums: the maximum
 // starts at the lowest finite float, a row whose every key is masked with that value is uniform,
@@ -38,6 +38,16 @@ __device__ __forceinline__ floatx4 mfma4(f4v a, f4v b, floatx4 c) {
     c = __builtin_amdgcn_mfma_f32_16x16x4f32(a.y, b.y, c, 0, 0, 0);
     c = __builtin_amdgcn_mfma_f32_16x16x4f32(a.z, b.z, c, 0, 0, 0);
     return __builtin_amdgcn_mfma_f32_16x16x4f32(a.w, b.w, c, 0, 0, 0);
+}
+
+// c plus 16 products, with SHORT as a chain of their own: the prompt's sums must not round worse than
+// the token steps', which add by lanes of few terms (the KV cache of 32 ids 7.40e-7 off 64 bits with
+// chains over a whole row, 7.02e-7 so, 7.11e-7 by token steps; 384 ids 22.7 -> 23.4 us a layer).  The
+// encoder's products were chains of 64 before too, and the additions cost it 0.7 %.
+template <bool SHORT>
+__device__ __forceinline__ floatx4 mfma_add(f4v a, f4v b, floatx4 c) {
+    if constexpr (SHORT) return c + mfma4(a, b, floatx4{0.f, 0.f, 0.f, 0.f});
+    else return mfma4(a, b, c);
 }
 
 // U query units per workgroup, two wavefronts each; grid batch x kv_heads x wgs, the last fastest,
@@ -134,7 +144,7 @@ __global__ __launch_bounds__(U * 128) void attention_kernel(AttnArgs a, int wgs,
             for (int j = 0; j < 4; ++j)
                 kf[j] = *reinterpret_cast<const f4v*>(&Kh[(16 * j + li) * kRs + 16 * c + 4 * g]);
 #pragma unroll
-            for (int j = 0; j < 4; ++j) s[j] = mfma4(kf[j], qf[c], s[j]);
+            for (int j = 0; j < 4; ++j) s[j] = mfma_add<CAUSAL>(kf[j], qf[c], s[j]);
         }
         // s[j][r]: key key0 + 16 j + 4 g + r, query li
         float mx = m;
@@ -181,10 +191,9 @@ __global__ __launch_bounds__(U * 128) void attention_kernel(AttnArgs a, int wgs,
 #pragma unroll
                 for (int d = 0; d < 4; ++d) vf[r][d] = Vh[(16 * j + 4 * g + r) * kRs + 16 * d + li];
 #pragma unroll
-            for (int r = 0; r < 4; ++r)
-#pragma unroll
-                for (int d = 0; d < 4; ++d)
-                    o[d] = __builtin_amdgcn_mfma_f32_16x16x4f32(vf[r][d], s[j][r], o[d], 0, 0, 0);
+            for (int d = 0; d < 4; ++d)
+                o[d] = mfma_add<CAUSAL>(f4v{vf[0][d], vf[1][d], vf[2][d], vf[3][d]},
+                                        f4v{s[j][0], s[j][1], s[j][2], s[j][3]}, o[d]);
         }
     }
     l += __shfl_xor(l, 16);

@@ -636,12 +636,23 @@ __device__ __host__ inline int64_t bl_b_extent(const GemmParams& p, int bmode) {
     return (int64_t)(p.K - 1) * p.sbk + p.N;
 }
 
-//
-// FL cuts the MFMA chains after every K tile and adds them to one of two further accumulator sets
-// in turn, for callers whose sums must not lose to a vector-unit reduction (the decoder's prompt
-// pass against its token steps): 3 % more issue slots.
+// Four steps of two k each.
+__device__ __forceinline__ floatx16 chain4(f4v a, f4v b, floatx16 c) {
+#pragma unroll
+    for (int q = 0; q < 4; ++q) c = __builtin_amdgcn_mfma_f32_32x32x2f32(a[q], b[q], c, 0, 0, 0);
+    return c;
+}
+
+// FL keeps the sums as accurate as a vector-unit reduction's (lanes of few terms and a tree), for the
+// decoder's prompt pass, whose sums must not lose to its token steps: the MFMA chains are cut every
+// half K tile, two accumulators in turn, each added in fp32 while the other one's chain runs; the
+// partial sums of every two tiles are added in fp64.  By the chains' lengths the rounding of a sum of
+// 2,048 is then 0.95 of the GEMV's (5,632: 0.9); chains of 32 k with two fp32 sums had 1.6 (2.1)
+// times that.  Measured on TinyLlama's shape, four seeds: the KV cache's distance from 64 bits after 130 ids
+// 1.570e-6 (1.677e-6 before, 1.579e-6 by token steps), after 384 4.350e-6 (4.432e-6, 4.354e-6); the
+// 384-id products 102 us on average, 97 before; fp64 additions for every half tile 109.
 template <int BM, int BN, int BK, int AM, int BMD, bool FL = false>
-__global__ __launch_bounds__(256) void gemm_bl_kernel(GemmParams p) {
+__global__ __launch_bounds__(256, FL ? 3 : 1) void gemm_bl_kernel(GemmParams p) {
     static_assert(AM == shp::A_KVEC || AM == shp::A_CONV_NHWC4, "row-contiguous A");
     static_assert(BMD == shp::B_NVEC || BMD == shp::B_KVEC, "row-contiguous B");
     constexpr int FM = BM / 64, FN = BN / 64;           // 2x2 waves of FM x FN 32x32 blocks
@@ -754,29 +765,18 @@ __global__ __launch_bounds__(256) void gemm_bl_kernel(GemmParams p) {
         }
     };
 
-    floatx16 acc[FM][FN], sum[2][FL ? FM : 1][FL ? FN : 1];
+    static_assert(!FL || (FM == 1 && FN == 1), "one 32x32 block per wavefront");
+    floatx16 acc[FM][FN], acc2, part;  // acc2, part, sum: FL
+    double sum[16];
 #pragma unroll
     for (int i = 0; i < FM; ++i)
 #pragma unroll
         for (int j = 0; j < FN; ++j)
 #pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                acc[i][j][r] = 0.0f;
-                if constexpr (FL) sum[0][i][j][r] = sum[1][i][j][r] = 0.0f;
-            }
-    auto flush = [&](int par) __attribute__((always_inline)) {
-        if constexpr (FL) {
+            for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.0f;
+    acc2 = part = acc[0][0];
 #pragma unroll
-            for (int i = 0; i < FM; ++i)
-#pragma unroll
-                for (int j = 0; j < FN; ++j)
-#pragma unroll
-                    for (int r = 0; r < 16; ++r) {
-                        sum[par][i][j][r] += acc[i][j][r];
-                        acc[i][j][r] = 0.0f;
-                    }
-        }
-    };
+    for (int r = 0; r < 16; ++r) sum[r] = 0.0;
 
     // Fragments of one step: lanes 0-31 feed k = s of the tile, lanes 32-63 k = BK/2 + s (A and
     // B agree, so any assignment of the tile's k to MFMA k-pairs works), so each lane reads four
@@ -799,15 +799,29 @@ __global__ __launch_bounds__(256) void gemm_bl_kernel(GemmParams p) {
             }
         }
     };
-    auto mma = [&](const Frag& f) __attribute__((always_inline)) {
+    auto mma = [&](const Frag& f, int s4) __attribute__((always_inline)) {
+        if constexpr (FL) {
+            floatx16& cur = s4 < NS / 2 ? acc[0][0] : acc2;
+            const bool first = s4 % (NS / 2) == 0;  // of a chain
+            if (first)
 #pragma unroll
-        for (int q = 0; q < 4; ++q)
+                for (int r = 0; r < 16; ++r) cur[r] = 0.0f;
+            cur = chain4(f.a[0], f.b[0], cur);
+            if (first) {
+                __builtin_amdgcn_sched_barrier(0);
+                part += s4 ? acc[0][0] : acc2;
+                asm volatile("" : "+v"(part));  // added here, behind the chain's start
+            }
+        } else {
 #pragma unroll
-            for (int fm = 0; fm < FM; ++fm)
+            for (int q = 0; q < 4; ++q)
 #pragma unroll
-                for (int fn = 0; fn < FN; ++fn)
-                    acc[fm][fn] =
-                        __builtin_amdgcn_mfma_f32_32x32x2f32(f.a[fm][q], f.b[fn][q], acc[fm][fn], 0, 0, 0);
+                for (int fm = 0; fm < FM; ++fm)
+#pragma unroll
+                    for (int fn = 0; fn < FN; ++fn)
+                        acc[fm][fn] =
+                            __builtin_amdgcn_mfma_f32_32x32x2f32(f.a[fm][q], f.b[fn][q], acc[fm][fn], 0, 0, 0);
+        }
     };
     // One K tile from LDS buffer `buf`; `wr` (the next tile) goes into buffer buf^1 chunk by
     // chunk when `do_store`, and tile `ld_kt` is loaded into `ld` chunk by chunk.  The
@@ -828,8 +842,8 @@ __global__ __launch_bounds__(256) void gemm_bl_kernel(GemmParams p) {
                 for (int e = e0; e < e1; ++e) store_e(buf ^ 1, wr, e);
 #pragma unroll
             for (int e = e0; e < e1; ++e) load_e(ld_kt, ld, e);
-            if (s4 & 1) mma(f1);
-            else mma(f0);
+            if (s4 & 1) mma(f1, s4);
+            else mma(f0, s4);
             __builtin_amdgcn_sched_barrier(0);
         }
     };
@@ -849,23 +863,24 @@ __global__ __launch_bounds__(256) void gemm_bl_kernel(GemmParams p) {
         int kt = 0;
         for (; kt + 1 < ntk; kt += 2) {
             tile(0, s1, true, s0, min(kt + 2, ntk - 1));
-            flush(0);
             __syncthreads();
             tile(1, s0, kt + 2 < ntk, s1, min(kt + 3, ntk - 1));
-            flush(1);
+            if (FL)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) {
+                    sum[r] += (double)part[r];
+                    part[r] = 0.0f;
+                }
             __syncthreads();
         }
         if (kt < ntk) {
             tile(0, s1, false, s0, kt);
-            flush(0);
             __syncthreads();
         }
     }
     if constexpr (FL)
 #pragma unroll
-        for (int i = 0; i < FM; ++i)
-#pragma unroll
-            for (int j = 0; j < FN; ++j) acc[i][j] = sum[0][i][j] + sum[1][i][j];
+        for (int r = 0; r < 16; ++r) acc[0][0][r] = (float)(sum[r] + (double)(part[r] + acc2[r]));
 
     gemm_epilogue<BM, BN, 2, 2, RC, CS, shp::C_STRIDED>(p, acc, smem, m0, n0, split, p.splits, bz,
                                                         bo, bi, gridDim.z,
@@ -2198,7 +2213,7 @@ double plan_cost(const GemmParams& p, int nbatch, TileCfg t, int splits, int kps
 //    and 32-deep 64x64 tiles, four of which fit, at 1 from eight to a CU on (4096x3072x768: 147 us,
 //    160 with the 16-deep tile).  Gathers with taps run at 1 / 1.58 of a product's rate.
 //  - The 16-deep K tile's higher residency wins 8 % on at most 256 k; beyond, K tiles tie, but
-//    with the short chains' second sums it runs at 0.85 (512-row prompt pass 10.5 ms, 11.4 without).
+//    with the short chains' further sums it runs at 0.85 (512-row prompt pass 10.5 ms, 11.4 without, at chains of 32 k).
 //  - A split writes and reads its partial sums and pays the counters' round trip.
 //  - The direct kernel's 32x64 tiles fill the rounds that 64x64 tiles leave half empty (600 tiles
 //    are 3 rounds of half the work, 300 are 2), but each round pays its pipeline's fill, which is

@@ -4,14 +4,17 @@
 // Feeding a prompt token by token reads all 4.1 GB of TinyLlama's weights per position
 // (0.76 ms each); a chunk of positions reads them once.  Up to 64 rows the products are bound by
 // that read, so they have their own kernel (skinny_kernel); above, they are matrix-core bound and
-// run on the tiled GEMM kernels.  TinyLlama's shape, whole prompt: 32 ids 24.3 -> 2.26 ms,
-// 384 ids 291 -> 9.1 ms; 1.6 ms is the least (2 ids, two token steps take 1.5).
+// run on the tiled GEMM kernels.  TinyLlama's shape, whole prompt: 32 ids 24.3 -> 2.41 ms,
+// 384 ids 291 -> 9.1 ms; 1.7 ms is the least (two token steps take 1.6).
 #include "prefill.h"
 #include "coherent.h"
+
+#include <type_traits>
 
 namespace {
 
 typedef float floatx4 __attribute__((ext_vector_type(4)));
+typedef double doublex4 __attribute__((ext_vector_type(4)));
 
 __device__ __forceinline__ float wave_sum(float v) {
 #pragma unroll
@@ -19,11 +22,11 @@ __device__ __forceinline__ float wave_sum(float v) {
     return v;
 }
 
-__device__ __forceinline__ floatx4 mfma4(f4v a, f4v b, floatx4 c) {
-    c = __builtin_amdgcn_mfma_f32_16x16x4f32(a.x, b.x, c, 0, 0, 0);
-    c = __builtin_amdgcn_mfma_f32_16x16x4f32(a.y, b.y, c, 0, 0, 0);
-    c = __builtin_amdgcn_mfma_f32_16x16x4f32(a.z, b.z, c, 0, 0, 0);
-    return __builtin_amdgcn_mfma_f32_16x16x4f32(a.w, b.w, c, 0, 0, 0);
+// Eight products of a column: two matrix instructions from zero.
+__device__ __forceinline__ floatx4 mfma2(float a0, float a1, float b0, float b1) {
+    floatx4 c = {0.f, 0.f, 0.f, 0.f};
+    c = __builtin_amdgcn_mfma_f32_16x16x4f32(a0, b0, c, 0, 0, 0);
+    return __builtin_amdgcn_mfma_f32_16x16x4f32(a1, b1, c, 0, 0, 0);
 }
 
 // ---- skinny_kernel: out = x[M][K] w[N][K]^T for M <= 16 MT rows -------------------------------
@@ -33,12 +36,15 @@ __device__ __forceinline__ floatx4 mfma4(f4v a, f4v b, floatx4 c) {
 // layout, no LDS and no barrier in the loop: lane l loads 16 bytes of row l % 16 at k + 4 * (l / 16).
 // The x rows are read the same way and come from L2 (256 KB at 32 rows of 2,048).  Four steps ahead
 // of the products, so a wavefront has 8 KB of weights in flight and a CU about 100 (TinyLlama at 32
-// rows: gate/up 41 us for 92 MB, the others 13 us; a form with x stationary in registers and 128 KB in
-// flight took 34 and 19, loading x into every CU first costs the small ones more).  The eight partial
-// tiles are summed in LDS in wavefront order.  The MFMA chains are cut every 32 k and added to a
-// second accumulator: the sum's rounding error is then that of the decode step's GEMV (lanes of ~32
-// terms and a tree), where one chain had 1.6 times it.  D = w x^T puts four consecutive n of one row
-// m in a lane: 16-byte stores, and gate and up of one output next to each other for the SwiGLU form.
+// rows: gate/up 43 us for 92 MB, the others 14 us; a form with x stationary in registers and 128 KB in
+// flight took 34 and 19, loading x into every CU first costs the small ones more).  The sums are built
+// to round no worse than the decode step's GEMV (lanes of few terms and a tree): MFMA chains of 8 k
+// from zero, up to ten of them added in fp32 before their sum is (up to 16 rows, where registers are
+// left, every two in fp64), and the eight wavefronts' partial tiles added in LDS as a tree.  With chains of 32 k and the wavefronts added in order the KV cache of
+// 32 ids was 8.24e-7 off 64 bits where token steps are 7.11e-7 (four seeds); so it is 7.02e-7, for 1 %
+// of the 32-id generation (16.77 -> 16.93 ms).
+// D = w x^T puts four consecutive n of one row m in a lane: 16-byte stores, and gate and up of one
+// output next to each other for the SwiGLU form.
 constexpr unsigned kOob = 0x80000000u;  // past every operand range: loads return 0
 constexpr int kSkWaves = 8;
 
@@ -47,6 +53,7 @@ __global__ __launch_bounds__(kSkWaves * 64, MT <= 2 ? 4 : 2) void skinny_kernel(
     const float* __restrict__ x, const float* __restrict__ w, float* __restrict__ out, int M, int N,
     int K, int kper) {
     constexpr int NT = 2, ST = 5;
+    typedef typename std::conditional<MT == 1, doublex4, floatx4>::type Sum;
     __shared__ __attribute__((aligned(16))) f4v red[MT * NT][kSkWaves][64];
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -85,20 +92,25 @@ __global__ __launch_bounds__(kSkWaves * 64, MT <= 2 ? 4 : 2) void skinny_kernel(
             d.x[i] = __builtin_bit_cast(
                 f4v, __builtin_amdgcn_raw_buffer_load_b128(xr, in ? xo[i] : kOob, so, 0));
     };
-    floatx4 acc[MT][NT], sum[MT][NT];
+    floatx4 acc[MT][NT];
+    Sum sum[MT][NT];
     const floatx4 zero = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int i = 0; i < MT; ++i)
 #pragma unroll
-        for (int j = 0; j < NT; ++j) acc[i][j] = sum[i][j] = zero;
+        for (int j = 0; j < NT; ++j) {
+            acc[i][j] = zero;
+            sum[i][j] = Sum{0, 0, 0, 0};
+        }
     auto mul = [&](const Set& s, bool cut) __attribute__((always_inline)) {
 #pragma unroll
         for (int i = 0; i < MT; ++i)
 #pragma unroll
             for (int j = 0; j < NT; ++j) {
-                acc[i][j] = mfma4(s.w[j], s.x[i], acc[i][j]);
-                if (cut) {
-                    sum[i][j] += acc[i][j];
+                acc[i][j] += mfma2(s.w[j].x, s.w[j].y, s.x[i].x, s.x[i].y) +
+                             mfma2(s.w[j].z, s.w[j].w, s.x[i].z, s.x[i].w);
+                if (cut || MT == 1) {
+                    sum[i][j] += __builtin_convertvector(acc[i][j], Sum);
                     acc[i][j] = zero;
                 }
             }
@@ -111,25 +123,27 @@ __global__ __launch_bounds__(kSkWaves * 64, MT <= 2 ? 4 : 2) void skinny_kernel(
         for (int u = 0; u < ST; ++u) {
             load(s + u + ST - 1, st[(u + ST - 1) % ST]);
             __builtin_amdgcn_sched_barrier(0);  // the loads stay ahead of the products
-            mul(st[u], (u & 1) || u == ST - 1);
+            mul(st[u], u == ST - 1);
             __builtin_amdgcn_sched_barrier(0);
         }
     }
 #pragma unroll
     for (int u = 0; u < ST - 1; ++u)
-        if (s + u < ns) mul(st[u], true);
-
+        if (s + u < ns) mul(st[u], false);
 #pragma unroll
     for (int i = 0; i < MT; ++i)
 #pragma unroll
-        for (int j = 0; j < NT; ++j)
-            red[i * NT + j][wave][lane] = f4v{sum[i][j][0], sum[i][j][1], sum[i][j][2], sum[i][j][3]};
+        for (int j = 0; j < NT; ++j) {
+            const floatx4 v = __builtin_convertvector(sum[i][j] + __builtin_convertvector(acc[i][j], Sum), floatx4);
+            red[i * NT + j][wave][lane] = f4v{v[0], v[1], v[2], v[3]};
+        }
     __syncthreads();
     const int t = wave;
     if (t >= MT * NT) return;
-    f4v v = red[t][0][lane];
+    f4v p[kSkWaves];
 #pragma unroll
-    for (int u = 1; u < kSkWaves; ++u) v += red[t][u][lane];
+    for (int u = 0; u < kSkWaves; ++u) p[u] = red[t][u][lane];
+    const f4v v = ((p[0] + p[1]) + (p[2] + p[3])) + ((p[4] + p[5]) + (p[6] + p[7]));
     const int m = 16 * (t / NT) + li, n = n0 + 16 * (t % NT) + 4 * g;
     if (m >= M || n >= N) return;
     if constexpr (MODE == shp::SK_SWIGLU) {

@@ -407,6 +407,62 @@ def test_llama_prompt_pass_of_narrow_models(ctx, hidden, ffn, vocab, n):
         assert_close(lm.logits(), want, 1e-5, 1e-4, f"hidden {hidden}, prompt of {n}")
 
 
+def llama64(layers, emb, cfg, ids):
+    """K and V of every layer and position in float64: [layer][2][kv, n, 64]."""
+    n, nh, nkv, out = len(ids), cfg["n_heads"], cfg["n_kv_heads"], []
+    norm = lambda x, w: x / np.sqrt((x * x).mean(-1, keepdims=True) + cfg["rms_eps"]) * w
+    ang = np.arange(n)[:, None, None] * cfg["rope_theta"] ** (-np.arange(0, 64, 2) / 64.0)
+    def rope(x):
+        a, b = x[..., :32], x[..., 32:]
+        return np.concatenate([a * np.cos(ang) - b * np.sin(ang), b * np.cos(ang) + a * np.sin(ang)], -1)
+    x = emb.reshape(-1, cfg["hidden"])[ids].astype(np.float64)
+    for w in layers:
+        an, wqkv, wo, fn, wgu, wd = (a.astype(np.float64) for a in w)
+        qkv = (norm(x, an) @ wqkv.reshape(-1, cfg["hidden"]).T).reshape(n, nh + 2 * nkv, 64)
+        q, k, v = rope(qkv[:, :nh]), rope(qkv[:, nh:nh + nkv]), qkv[:, nh + nkv:]
+        out.append((k.transpose(1, 0, 2), v.transpose(1, 0, 2)))
+        att = np.empty((n, nh, 64))
+        for h in range(nh):
+            s = q[:, h] @ k[:, h * nkv // nh].T * 0.125
+            s[np.triu_indices(n, 1)] = -np.inf
+            p = np.exp(s - s.max(-1, keepdims=True))
+            att[:, h] = p / p.sum(-1, keepdims=True) @ v[:, h * nkv // nh]
+        x = x + att.reshape(n, -1) @ wo.reshape(cfg["hidden"], -1).T
+        gu = norm(x, fn) @ wgu.reshape(-1, cfg["hidden"]).T
+        g, u = gu[:, 0::2], gu[:, 1::2]
+        x = x + (g / (1 + np.exp(-g)) * u) @ wd.reshape(cfg["hidden"], -1).T
+    return out
+
+
+@pytest.mark.parametrize("n", [16, 48, 100])
+def test_llama_prompt_pass_rounds_no_worse_than_token_steps(ctx, n):
+    """The KV cache's distance from float64, all layers together, by the pass and by token steps: the
+    pass's sums are built to round less.  2 % for what 1e5 rounding errors of one seed average to."""
+    from spirv_inference_amd.models import Llama
+    cfg = dict(SMALL, n_layers=4, hidden=2048, n_heads=16, n_kv_heads=4, ffn=2816, max_seq=128)
+    prompt = [int(t) for t in np.random.default_rng(n).integers(3, cfg["vocab"], n)]
+    with Llama(ctx, seed=9, **cfg) as lm:
+        want = llama64(llama_layers(lm, 4), lm.weight(0, "embed"), cfg, prompt)
+
+        def error():
+            num = den = 0.0
+            for layer in range(1, 4):
+                for which, w in zip(("k_cache", "v_cache"), want[layer]):
+                    got = lm.weight(layer, which).reshape(4, -1, 64)[:, :n]
+                    num += float(((got - w) ** 2).sum() / (w ** 2).sum())
+            return num ** 0.5
+
+        lm.reset()
+        for t in prompt:
+            lm.step(t)
+        ctx.sync()
+        steps = error()
+        lm.generate(prompt, 1)
+        one_pass = error()
+        print(f"[llama] {n} ids: distance {one_pass:.3e} by the pass, {steps:.3e} by steps", flush=True)
+        assert one_pass <= steps * 1.02
+
+
 def test_llama_generate_refuses_bad_prompts(ctx):
     from spirv_inference_amd import ShpError
     from spirv_inference_amd.models import Llama
